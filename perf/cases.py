@@ -404,9 +404,9 @@ def work(case):
 
 def tolerance(case):
     """f32 sums in another order: about four times the error measured against 64 bits.  A layer's steps, and a
-    model's layers above all, carry a change of rounding on."""
+    model's layers above all, carry a change of rounding on (the decode's is measured between two orders of its sums)."""
     return {"rel": {"matvec": 1e-6, "packed": 1e-6, "matmul": 1e-6, "attention": 4e-6, "layer": 4e-6, "prompt": 2e-5,
-                    "chat": 2e-5, "decode": 2e-4}[case["kind"]]}
+                    "chat": 2e-5, "decode": 5e-6}[case["kind"]]}
 
 
 # --------------------------------------------------------------------- exact

@@ -356,8 +356,8 @@ int32_t rf_model_kv_capacity(rf_model *model, uint64_t *tokens);
 /* Which kernels the model runs (no counterpart in the reference, which has
  * one CPU path; for tests and tools that must know which path they cover):
  * split_attention = 1 when decode attention runs the split-K kernel
- * (32/8/... query-KV head ratios with head_dim 64, 128 or 256), 0 for the
- * any-shape kernel; regime = the split kernel's launch regime (0-4) of a
+ * (a whole number of query heads per KV head with head_dim 64, 96, 128 or
+ * 256), 0 for the any-shape kernel; regime = the split kernel's launch regime (0-4) of a
  * decode step at position pos (0 for the any-shape kernel);
  * batched_prefill = 1 when rf_model_prefill (and rf_model_generate after
  * rf_model_set_prefill(1)) forwards prompts as batched GEMMs with the

@@ -98,15 +98,22 @@ __device__ __forceinline__ void load_few(float* dst, const float* src) {
   }
 }
 
-// n dims of a K row for one lane: four consecutive floats from every 64
-// (src points at the lane's first float of the row).
-__device__ __forceinline__ void load_dims(float* dst, const float* src, int n) {
-  const f32x4* p = reinterpret_cast<const f32x4*>(src);
+// A K row's dims over the 16 lanes of a position: lane sl holds dims
+// 16 V (i / V) + V sl + i % V, i < hd / 16, so each of a lane's loads takes V
+// floats and the 16 lanes of one load read 64 V contiguous bytes (V = 4
+// where head_dim is a multiple of 64, 2 for 96).
+template <int HD> constexpr int att_vec() { return HD % 64 == 0 ? 4 : HD % 32 == 0 ? 2 : 1; }
+template <int HD> __device__ __forceinline__ uint32_t att_dim(uint32_t sl, int i) {
+  constexpr int V = att_vec<HD>();
+  return 16u * V * (i / V) + V * sl + i % V;
+}
+
+// The dims of a K or V row for one lane (src points at the lane's first float of the row).
+template <int HD>
+__device__ __forceinline__ void load_dims(float* dst, const float* src) {
+  constexpr int V = att_vec<HD>();
 #pragma unroll
-  for (int i = 0; i < n / 4; ++i) {
-    const f32x4 v = __builtin_nontemporal_load(p + 16 * i);
-    dst[4 * i] = v.x; dst[4 * i + 1] = v.y; dst[4 * i + 2] = v.z; dst[4 * i + 3] = v.w;
-  }
+  for (int i = 0; i < HD / 16 / V; ++i) load_few<V>(dst + V * i, src + 16 * V * i);
 }
 
 // Raw buffer loads over one chunk's rows of one KV head: offsets past the
@@ -117,16 +124,6 @@ constexpr int ATT_RSRC_WORD3 = 0x00020000;  // raw buffer, 32-bit data
 constexpr int ATT_AUX_NT = 2;               // streaming loads
 __device__ __forceinline__ AttRsrc att_rsrc(const float* base, uint32_t bytes) {
   return __builtin_amdgcn_make_buffer_rsrc(const_cast<float*>(base), 0, (int32_t)bytes, ATT_RSRC_WORD3);
-}
-// n dims of a K row for one lane (four consecutive floats from every 64) at
-// byte offset off of the region
-__device__ __forceinline__ void load_dims_buf(float* dst, AttRsrc r, uint32_t off, int n) {
-#pragma unroll
-  for (int i = 0; i < n / 4; ++i) {
-    const auto v = __builtin_amdgcn_raw_buffer_load_b128(r, off + 256u * i, 0, ATT_AUX_NT);
-    dst[4 * i] = __uint_as_float(v[0]); dst[4 * i + 1] = __uint_as_float(v[1]);
-    dst[4 * i + 2] = __uint_as_float(v[2]); dst[4 * i + 3] = __uint_as_float(v[3]);
-  }
 }
 template <int N>
 __device__ __forceinline__ void load_few_buf(float* dst, AttRsrc r, uint32_t off) {
@@ -140,6 +137,13 @@ __device__ __forceinline__ void load_few_buf(float* dst, AttRsrc r, uint32_t off
 #pragma unroll
     for (int i = 0; i < 4; ++i) dst[i] = __uint_as_float(v[i]);
   }
+}
+// load_dims at byte offset off of the region
+template <int HD>
+__device__ __forceinline__ void load_dims_buf(float* dst, AttRsrc r, uint32_t off) {
+  constexpr int V = att_vec<HD>();
+#pragma unroll
+  for (int i = 0; i < HD / 16 / V; ++i) load_few_buf<V>(dst + V * i, r, off + 64u * V * i);
 }
 
 // W wavefronts per workgroup: one round of loads covers 16 W positions
@@ -158,7 +162,9 @@ __global__ __launch_bounds__(64 * W) void attn_split(AttnArgs a) {
   constexpr uint32_t RV = 16;                                 // V rows per wavefront and round
   // (Holding a whole 256-position chunk in flight, 8 K positions per lane
   // and 32 V rows per wavefront, measured slower at 2048-8000 positions.)
-  constexpr uint32_t WMASK = 16u / G - 1u;
+  // a group of 3, 5, 6 or 7 heads is summed as 4 or 8 with zeros beyond it
+  constexpr int GP = G <= 2 ? G : G <= 4 ? 4 : 8;
+  constexpr uint32_t WMASK = 16u / GP - 1u;
   __shared__ __align__(16) float sc[G][ATT_MAX_CHUNK];
   __shared__ __align__(16) float qs[G][HD];
   __shared__ __align__(16) float kcur[HD];
@@ -192,18 +198,20 @@ __global__ __launch_bounds__(64 * W) void attn_split(AttnArgs a) {
   const uint32_t ns = (total + chunk - 1) / chunk;
   const float* cs = a.rope ? a.rope + (size_t)hist * HD : nullptr;  // [half][2] for this position
   const uint32_t sl = lane & 15u, slot = wave * 4u + (lane >> 4);
-  // Lane sl of a position holds dims kdim(i) = 64 (i / 4) + 4 sl + i % 4, so
-  // each 16-byte load of the 16 lanes covers 256 contiguous bytes of the row.
-  const uint32_t d0 = sl * 4u;
+  const uint32_t d0 = att_dim<HD>(sl, 0);
   // K and V rows p0 .. p0 + nmain - 1 of KV head g: a region ending with the
   // last row's head segment; rows past it (a round's tail) read as zeros
   const uint32_t rbytes = nmain ? ((nmain - 1u) * kvw + HD) * 4u : 0u;
   const AttRsrc kr = att_rsrc(a.k_hist + (size_t)p0 * kvw + g * HD, rbytes);
   const AttRsrc vr = att_rsrc(a.v_hist + (size_t)p0 * kvw + g * HD, rbytes);
   // Pass 2 maps lanes to dims instead: lane l owns dims [l*DPW, (l+1)*DPW) of
-  // every V row and wavefront w the rows w*16 .. w*16+15 of each 64-row batch,
-  // so the weighted V sum needs no cross-lane reduction.
-  constexpr int DPW = HD / 64;
+  // every V row (lanes past the row none: they read dim 0 and write nothing)
+  // and wavefront w the rows w*16 .. w*16+15 of each 64-row batch, so the
+  // weighted V sum needs no cross-lane reduction.
+  constexpr int DPW = (HD + 63) / 64;
+  static_assert(HD % DPW == 0, "whole lanes");
+  const bool vlane = HD % 64 == 0 || lane * DPW < (uint32_t)HD;
+  const uint32_t vd0 = vlane ? lane * DPW : 0u;
 
   // Loads first: the prologue's operands (q of the G heads, the current k
   // and v, the cos/sin row), then the first batch of K rows, then of V rows,
@@ -227,10 +235,10 @@ __global__ __launch_bounds__(64 * W) void attn_split(AttnArgs a) {
   __builtin_amdgcn_sched_barrier(0);
   float kv[U][DPL], vv[RV][DPW];
 #pragma unroll
-  for (int u = 0; u < U; ++u) load_dims_buf(kv[u], kr, ((slot + NSLOT * u) * kvw + d0) * 4u, DPL);
+  for (int u = 0; u < U; ++u) load_dims_buf<HD>(kv[u], kr, ((slot + NSLOT * u) * kvw + d0) * 4u);
   __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-  for (int k = 0; k < (int)RV; ++k) load_few_buf<DPW>(vv[k], vr, ((wave * RV + k) * kvw + lane * DPW) * 4u);
+  for (int k = 0; k < (int)RV; ++k) load_few_buf<DPW>(vv[k], vr, ((wave * RV + k) * kvw + vd0) * 4u);
   __builtin_amdgcn_sched_barrier(0);
 
   // Rotated q of the G heads, the current k (rotated) and v, and the slot write.
@@ -257,42 +265,46 @@ __global__ __launch_bounds__(64 * W) void attn_split(AttnArgs a) {
 #pragma unroll
   for (int h = 0; h < G; ++h)
 #pragma unroll
-    for (int i = 0; i < DPL; ++i) qr[h][i] = qs[h][64 * (i / 4) + d0 + i % 4];
+    for (int i = 0; i < DPL; ++i) qr[h][i] = qs[h][att_dim<HD>(sl, i)];
 
   // Pass 1: scores.
   for (uint32_t j0 = 0; j0 < nmain; j0 += NSLOT * U) {
     if (j0 > 0) {
 #pragma unroll
-      for (int u = 0; u < U; ++u) load_dims_buf(kv[u], kr, ((j0 + slot + NSLOT * u) * kvw + d0) * 4u, DPL);
+      for (int u = 0; u < U; ++u) load_dims_buf<HD>(kv[u], kr, ((j0 + slot + NSLOT * u) * kvw + d0) * 4u);
     }
 #pragma unroll
     for (int u = 0; u < U; ++u) {
-      float s[G];
+      float s[GP];
 #pragma unroll
-      for (int h = 0; h < G; ++h) {
+      for (int h = 0; h < GP; ++h) {
         float acc = 0.f;
+        if (h < G) {
 #pragma unroll
-        for (int i = 0; i < DPL; ++i) acc = fmaf(qr[h][i], kv[u][i], acc);
+          for (int i = 0; i < DPL; ++i) acc = fmaf(qr[h][i], kv[u][i], acc);
+        }
         s[h] = acc;
       }
       uint32_t hh = 0;
-      const float r = head_reduce16<G, 8>(s, lane, hh);
+      const float r = head_reduce16<GP, 8>(s, lane, hh);
       const uint32_t j = j0 + slot + NSLOT * u;
-      if (j < nmain && (lane & WMASK) == 0) sc[hh][j] = r / a.denom;
+      if (j < nmain && (lane & WMASK) == 0 && hh < (uint32_t)G) sc[hh][j] = r / a.denom;
     }
   }
   if (has_cur && wave == 0) {
-    float s[G];
+    float s[GP];
 #pragma unroll
-    for (int h = 0; h < G; ++h) {
+    for (int h = 0; h < GP; ++h) {
       float acc = 0.f;
+      if (h < G) {
 #pragma unroll
-      for (int i = 0; i < DPL; ++i) acc = fmaf(qr[h][i], kcur[64 * (i / 4) + d0 + i % 4], acc);
+        for (int i = 0; i < DPL; ++i) acc = fmaf(qr[h][i], kcur[att_dim<HD>(sl, i)], acc);
+      }
       s[h] = acc;
     }
     uint32_t hh = 0;
-    const float r = head_reduce16<G, 8>(s, lane, hh);
-    if (slot == 0 && (lane & WMASK) == 0) sc[hh][nmain] = r / a.denom;
+    const float r = head_reduce16<GP, 8>(s, lane, hh);
+    if (slot == 0 && (lane & WMASK) == 0 && hh < (uint32_t)G) sc[hh][nmain] = r / a.denom;
   }
   __syncthreads();
 
@@ -328,7 +340,7 @@ __global__ __launch_bounds__(64 * W) void attn_split(AttnArgs a) {
   for (uint32_t j0 = 0; j0 < nmain; j0 += RV * W) {
     if (j0 > 0) {
 #pragma unroll
-      for (int k = 0; k < (int)RV; ++k) load_few_buf<DPW>(vv[k], vr, ((j0 + wave * RV + k) * kvw + lane * DPW) * 4u);
+      for (int k = 0; k < (int)RV; ++k) load_few_buf<DPW>(vv[k], vr, ((j0 + wave * RV + k) * kvw + vd0) * 4u);
     }
     // weights of this wavefront's rows, four at a time with 16-byte LDS reads
     // (j0 + RV w is a multiple of 16, and j0 + RV (w + 1) <= ATT_MAX_CHUNK
@@ -354,14 +366,15 @@ __global__ __launch_bounds__(64 * W) void attn_split(AttnArgs a) {
     for (int h = 0; h < G; ++h) {
       const float e = sc[h][nmain];
 #pragma unroll
-      for (int i = 0; i < DPW; ++i) o[h][i] = fmaf(e, vcur[lane * DPW + i], o[h][i]);
+      for (int i = 0; i < DPW; ++i) o[h][i] = fmaf(e, vcur[vd0 + i], o[h][i]);
     }
   }
   // Sum the W wavefronts.
 #pragma unroll
   for (int h = 0; h < G; ++h)
 #pragma unroll
-    for (int i = 0; i < DPW; ++i) ored[wave][h][lane * DPW + i] = o[h][i];
+    for (int i = 0; i < DPW; ++i)
+      if (vlane) ored[wave][h][vd0 + i] = o[h][i];
   __syncthreads();
   for (uint32_t t = tid; t < (uint32_t)(G * HD); t += NTH) {
     const uint32_t h = t / HD, d = t % HD;
@@ -420,7 +433,7 @@ __global__ __launch_bounds__(64 * W) void attn_flash(AttnArgs a) {
   const uint32_t ns = (total + chunk - 1) / chunk;
   const float* cs = a.rope ? a.rope + (size_t)hist * HD : nullptr;
   const uint32_t sl = lane & 15u, slot = wave * 4u + (lane >> 4);
-  const uint32_t d0 = sl * 4u;  // dims 64 (i / 4) + d0 + i % 4 of K and V rows
+  const uint32_t d0 = att_dim<HD>(sl, 0);
   const float* kb = a.k_hist + (size_t)p0 * kvw + g * HD + d0;
   const float* vb = a.v_hist + (size_t)p0 * kvw + g * HD + d0;
 
@@ -443,12 +456,12 @@ __global__ __launch_bounds__(64 * W) void attn_flash(AttnArgs a) {
 #pragma unroll
     for (int u = 0; u < U; ++u) {
       const uint32_t j = min(j0 + slot + NSLOT * u, nmain - 1u);
-      load_dims(kv[u], kb + (size_t)j * kvw, DPL);
+      load_dims<HD>(kv[u], kb + (size_t)j * kvw);
     }
 #pragma unroll
     for (int u = 0; u < U; ++u) {
       const uint32_t j = min(j0 + slot + NSLOT * u, nmain - 1u);
-      load_dims(vv[u], vb + (size_t)j * kvw, DPL);
+      load_dims<HD>(vv[u], vb + (size_t)j * kvw);
     }
   };
   if (nmain > 0) issue(0);
@@ -478,7 +491,7 @@ __global__ __launch_bounds__(64 * W) void attn_flash(AttnArgs a) {
 #pragma unroll
   for (int h = 0; h < G; ++h)
 #pragma unroll
-    for (int i = 0; i < DPL; ++i) qr[h][i] = qs[h][64 * (i / 4) + d0 + i % 4] * qscale;
+    for (int i = 0; i < DPL; ++i) qr[h][i] = qs[h][att_dim<HD>(sl, i)] * qscale;
   float m[G], l[G], o[G][DPL];
 #pragma unroll
   for (int h = 0; h < G; ++h) {
@@ -532,8 +545,8 @@ __global__ __launch_bounds__(64 * W) void attn_flash(AttnArgs a) {
     for (int u = 0; u < U; ++u)
 #pragma unroll
       for (int i = 0; i < DPL; ++i) {
-        kk[u][i] = kcur[64 * (i / 4) + d0 + i % 4];
-        vw[u][i] = vcur[64 * (i / 4) + d0 + i % 4];
+        kk[u][i] = kcur[att_dim<HD>(sl, i)];
+        vw[u][i] = vcur[att_dim<HD>(sl, i)];
       }
     consume(kk, vw, 0, 1);  // only slot 0, u = 0 is valid
   }
@@ -556,7 +569,7 @@ __global__ __launch_bounds__(64 * W) void attn_flash(AttnArgs a) {
 #pragma unroll
     for (int h = 0; h < G; ++h) {
 #pragma unroll
-      for (int i = 0; i < DPL; ++i) po[wave][h][64 * (i / 4) + d0 + i % 4] = o[h][i];
+      for (int i = 0; i < DPL; ++i) po[wave][h][att_dim<HD>(sl, i)] = o[h][i];
       if (lane == 0) { pm[wave][h] = m[h]; pl[wave][h] = l[h]; }
     }
   }
@@ -585,15 +598,20 @@ __global__ __launch_bounds__(64 * W) void attn_flash(AttnArgs a) {
 }
 
 // Merge the chunk records (o, m, l) of one query head: one wavefront per
-// head, lane l owning dims [l DPW, (l + 1) DPW).  The first 32 records (all
+// head, lane l owning dims [l DPW, (l + 1) DPW), DPW = ceil(HD / 64) (lanes
+// past the row none).  The first 32 records (all
 // of them up to 32 chunks) are requested together with the (m, l) pairs,
 // before any arithmetic; the factors exp(m_s - M) go through LDS to every
 // lane.
-template <int DPW>
+template <int HD>
 __global__ __launch_bounds__(64) void attn_merge(AttnArgs a) {
-  constexpr uint32_t HD = 64u * DPW, B = 32, MPL = ATT_MAX_SPLITS / 64;  // (m, l) pairs per lane
+  constexpr int DPW = (HD + 63) / 64;
+  static_assert(HD % DPW == 0, "whole lanes");
+  constexpr uint32_t B = 32, MPL = ATT_MAX_SPLITS / 64;  // (m, l) pairs per lane
   __shared__ float fac[ATT_MAX_SPLITS];
   const uint32_t qhead = blockIdx.x, lane = threadIdx.x;
+  const bool vlane = HD % 64 == 0 || lane * DPW < (uint32_t)HD;
+  const uint32_t vd0 = vlane ? lane * DPW : 0u;
   const uint32_t z = blockIdx.z;  // token batch: see attn_split
   const uint32_t hist = (a.d_pos ? (uint32_t)(*a.d_pos) : a.hist) + z;
   const uint32_t total = hist + 1;
@@ -604,7 +622,7 @@ __global__ __launch_bounds__(64) void attn_merge(AttnArgs a) {
   const float* base = a.ws + (size_t)z * a.nsplit * stride + (size_t)qhead * rec;
   float pre[B][DPW];
 #pragma unroll
-  for (uint32_t s = 0; s < B; ++s) load_few<DPW>(pre[s], base + (size_t)min(s, ns - 1u) * stride + lane * DPW);
+  for (uint32_t s = 0; s < B; ++s) load_few<DPW>(pre[s], base + (size_t)min(s, ns - 1u) * stride + vd0);
   float ms[MPL], ls[MPL];
 #pragma unroll
   for (uint32_t k = 0; k < MPL; ++k) {
@@ -640,7 +658,7 @@ __global__ __launch_bounds__(64) void attn_merge(AttnArgs a) {
   for (uint32_t s0 = B; s0 < ns; s0 += 16u) {
     float v[16][DPW];
 #pragma unroll
-    for (uint32_t j = 0; j < 16; ++j) load_few<DPW>(v[j], base + (size_t)min(s0 + j, ns - 1u) * stride + lane * DPW);
+    for (uint32_t j = 0; j < 16; ++j) load_few<DPW>(v[j], base + (size_t)min(s0 + j, ns - 1u) * stride + vd0);
 #pragma unroll
     for (uint32_t j = 0; j < 16; ++j)
       if (s0 + j < ns) {
@@ -648,7 +666,8 @@ __global__ __launch_bounds__(64) void attn_merge(AttnArgs a) {
         for (int i = 0; i < DPW; ++i) acc[i] = fmaf(fac[s0 + j], v[j][i], acc[i]);
       }
   }
-  float* o = a.out + (size_t)z * a.qh * HD + (size_t)qhead * HD + lane * DPW;
+  if (!vlane) return;
+  float* o = a.out + (size_t)z * a.qh * HD + (size_t)qhead * HD + vd0;
 #pragma unroll
   for (int i = 0; i < DPW; ++i) o[i] = acc[i] / l;
 }
@@ -897,14 +916,22 @@ __global__ __launch_bounds__(256) void attn_naive(AttnArgs a) {
   }
 }
 
+// The split kernels' shapes: any whole number of query heads per KV head with
+// head_dim 64, 96, 128 or 256.  attn_naive keeps the rest (other head_dims,
+// contexts of more than ATT_MAX_SPLITS chunks): its single workgroup per head
+// walks K and V column by column: 512 us against 9.5 us for 12 / 2 heads, hd
+// 128, 1501 positions; the 12 / 2 head Q4_0 chat turn of 203 prompt tokens and 6
+// more (8 layers of 1536) 150 ms against 5.1 ms, its prompt batched.
 bool attention_supported(uint32_t qh, uint32_t kvh, uint32_t hd, uint64_t total) {
   if (kvh == 0 || qh % kvh != 0) return false;
   if (total > (uint64_t)ATT_MAX_SPLITS * ATT_MAX_CHUNK) return false;
-  const uint32_t G = qh / kvh;
-  const bool g_ok = G == 1 || G == 2 || G == 4 || G == 8;
-  const bool hd_ok = hd == 64 || hd == 128 || hd == 256;
-  return g_ok && hd_ok && G * (hd / 16) <= 64;
+  return hd == 64 || hd == 96 || hd == 128 || hd == 256;
 }
+
+// A workgroup can take all G query heads of a KV head: G up to 8 while its q
+// and scores fit the registers.  Beyond (larger groups, hd 256 with G > 4)
+// every launch is per query head.
+bool attention_per_kv(uint32_t G, uint32_t hd) { return hd == 256 ? G == 1 || G == 2 || G == 4 : G >= 1 && G <= 8; }
 
 // Chunks per KV head: 64 positions each while that keeps the launch within
 // about 256 workgroups (one per CU), longer chunks beyond (at most
@@ -937,6 +964,8 @@ uint32_t attention_splits(uint32_t total, uint32_t kvh) {
 //   2  <= 128 Sq: per query head, 8 wavefronts (1024 positions: 9.6 vs 10.1);
 //   3  <= 64 Skv (Skv = attention_splits(cap)): per KV head, 4 wavefronts;
 //   4  beyond: per KV head, 8 wavefronts.
+// Shapes without a per-KV-head kernel (attention_per_kv) stay per query head
+// in 3 and 4, with Skv chunks counted over the query heads.
 // The workgroups of one chunk's query heads sit nsplit apart in dispatch
 // order, so with nsplit a multiple of 8 they land on one XCD and the re-reads
 // of that chunk's K/V by the G heads of a group hit its L2.  Past ~1K
@@ -947,8 +976,9 @@ static uint32_t regime_sq(uint32_t qh) {
   const uint32_t s = qh >= 256 ? 1u : 256u / qh;
   return s > 8 ? 8u : s;
 }
-static uint32_t regime_skv(uint64_t cap, uint32_t kvh) {
-  return attention_splits((uint32_t)(cap < 0xFFFFFFFFull ? cap : 0xFFFFFFFFull), kvh);
+static uint32_t regime_skv(uint64_t cap, uint32_t qh, uint32_t kvh, uint32_t hd) {
+  return attention_splits((uint32_t)(cap < 0xFFFFFFFFull ? cap : 0xFFFFFFFFull),
+                          attention_per_kv(kvh ? qh / kvh : 0, hd) ? kvh : qh);
 }
 // Regime 0's longest context (one chunk per query head, no merge): 64, or
 // rf_tune_attention_single's 128 / 256 (8 wavefronts above 64).  Timed in
@@ -959,23 +989,24 @@ static uint32_t g_single_max = ATT_MIN_CHUNK;
 void set_attention_single(uint32_t n) { g_single_max = n; }
 uint32_t attention_single() { return g_single_max; }
 
-AttnShape attention_regime_shape(int r, uint32_t qh, uint32_t kvh, uint64_t cap) {
+AttnShape attention_regime_shape(int r, uint32_t qh, uint32_t kvh, uint32_t hd, uint64_t cap) {
   const uint32_t sq = regime_sq(qh);
-  const uint32_t skv = regime_skv(cap, kvh);
+  const uint32_t skv = regime_skv(cap, qh, kvh, hd);
+  const uint32_t per_q = attention_per_kv(kvh ? qh / kvh : 0, hd) ? 0u : 1u;
   switch (r) {
     case 0: return AttnShape{1, 1, g_single_max > ATT_MIN_CHUNK ? 8u : 4u};
     case 1: return AttnShape{1, sq, 4};
     case 2: return AttnShape{1, sq, 8};
-    case 3: return AttnShape{0, skv, 4};
-    default: return AttnShape{0, skv, 8};
+    case 3: return AttnShape{per_q, skv, 4};
+    default: return AttnShape{per_q, skv, 8};
   }
 }
-int attention_regime(uint64_t total, uint32_t qh, uint32_t kvh, uint64_t cap) {
+int attention_regime(uint64_t total, uint32_t qh, uint32_t kvh, uint32_t hd, uint64_t cap) {
   const uint64_t sq = regime_sq(qh);
   if (total <= g_single_max) return 0;
   if (total <= ATT_MIN_CHUNK * sq) return 1;
   if (total <= 2 * ATT_MIN_CHUNK * sq) return 2;
-  return total <= ATT_MIN_CHUNK * (uint64_t)regime_skv(cap, kvh) ? 3 : 4;
+  return total <= ATT_MIN_CHUNK * (uint64_t)regime_skv(cap, qh, kvh, hd) ? 3 : 4;
 }
 
 uint64_t attention_ws_floats(uint32_t nsplit, uint32_t qh, uint32_t hd) {
@@ -998,9 +1029,12 @@ int attention_kernel() { return g_att_kernel; }
 
 template <int G, int DPL, int W, bool PERQ = false>
 static void launch_split_t(const AttnArgs& a, hipStream_t st) {
-  if (a.ntok == 0 && (g_att_kernel == 2 || (g_att_kernel == 1 && PERQ))) {
-    RF_KLAUNCH((attn_flash<G, DPL, W, PERQ>), dim3(a.nsplit, PERQ ? a.qh : a.kvh, 1), dim3(64 * W), 0, st, a);
-    return;
+  // mode 2 (experiments) knows groups of 1, 2, 4 and 8 heads per workgroup
+  if constexpr (PERQ || (DPL != 6 && (G & (G - 1)) == 0)) {
+    if (a.ntok == 0 && (g_att_kernel == 2 || (g_att_kernel == 1 && PERQ))) {
+      RF_KLAUNCH((attn_flash<G, DPL, W, PERQ>), dim3(a.nsplit, PERQ ? a.qh : a.kvh, 1), dim3(64 * W), 0, st, a);
+      return;
+    }
   }
   RF_KLAUNCH((attn_split<G, DPL, W, PERQ>), dim3(a.nsplit, PERQ ? a.qh : a.kvh, a.ntok ? a.ntok : 1),
                      dim3(64 * W), 0, st, a);
@@ -1022,8 +1056,7 @@ hipError_t launch_attention_naive(const AttnArgs& a, hipStream_t st) {
 }
 
 // Token batches on the matrix-core kernel (rf_tune_prefill_attention):
-// G = 1, 2, 4 or 8 query heads per KV head, head_dim 64 or 128, cache
-// offsets within 32 bits, and more than APF_MIN_TOTAL positions.  Timed on
+// up to 8 query heads per KV head, head_dim 64, 96 or 128, cache offsets within 32 bits, and more than APF_MIN_TOTAL positions.  Timed on
 // the 8B Q8_0 prompt (32 / 8 heads, hd 128), whole prompt: 8000 tokens
 // 998 ms against 1520 ms with the split kernel, 2048 tokens 209 against 224
 // ms, but 512 tokens 49.5 against 47.8 ms: for short contexts the split
@@ -1036,8 +1069,7 @@ int prefill_attention_mfma() { return g_apf; }
 bool prefill_attention_mfma_supported(uint32_t qh, uint32_t kvh, uint32_t hd, uint64_t total) {
   if (g_apf == 0 || kvh == 0 || qh % kvh || (g_apf == 1 && total <= APF_MIN_TOTAL)) return false;
   const uint32_t G = qh / kvh;
-  return (G == 1 || G == 2 || G == 4 || G == 8) && (hd == 64 || hd == 128) &&
-         total * kvh * hd * 4 < (1ull << 31);
+  return G >= 1 && G <= 8 && (hd == 64 || hd == 96 || hd == 128) && total * kvh * hd * 4 < (1ull << 31);
 }
 // Position splits of a prefill launch on that kernel: at least enough
 // workgroups (16-token tiles x KV heads x splits) for 256 CUs, and about 256
@@ -1045,10 +1077,10 @@ bool prefill_attention_mfma_supported(uint32_t qh, uint32_t kvh, uint32_t hd, ui
 // ATT_MIN_CHUNK positions give (att_chunk's smallest chunk).
 // Token tiles per workgroup: two for G <= 4 (the workgroup's K / V tiles
 // serve 32 tokens; 8000-token 8B prompt 965 against 997 ms with one), one
-// for G = 8 (512 threads already).
+// for larger groups (320 to 512 threads already).
 template <int G> constexpr int apf_tiles() { return G <= 4 ? 2 : 1; }
 uint32_t prefill_attention_mfma_splits(uint64_t total, uint64_t ntok, uint32_t kvh) {
-  const uint64_t per = APF_TOK * 2;  // workgroups of two token tiles (G = 8: one; more splits then)
+  const uint64_t per = APF_TOK * 2;  // workgroups of two token tiles (G > 4: one; more splits then)
   const uint64_t tiles = (ntok + per - 1) / per * (kvh ? kvh : 1);
   uint64_t n = (256 + tiles - 1) / tiles;
   const uint64_t by_len = (total + 255) / 256, most = (total + ATT_MIN_CHUNK - 1) / ATT_MIN_CHUNK;
@@ -1065,69 +1097,90 @@ static void launch_apf_t(const AttnArgs& a, hipStream_t st) {
              dim3(64 * G * TT), 0, st, a);
 }
 
+template <int G>
+static void launch_apf_g(const AttnArgs& a, hipStream_t st) {
+  if (a.hd == 64) launch_apf_t<G, 64>(a, st);
+  else if (a.hd == 96) launch_apf_t<G, 96>(a, st);
+  else launch_apf_t<G, 128>(a, st);
+}
+
+// The merge of the chunk records the launch before left (its own error first).
+static hipError_t launch_merge(const AttnArgs& a, hipStream_t st) {
+  const hipError_t e = hipGetLastError();
+  if (e != hipSuccess || a.nsplit == 1 || a.defer_merge) return e;
+  const dim3 mg(a.qh, 1, a.ntok ? a.ntok : 1);
+  switch (a.hd) {
+    case 64: RF_KLAUNCH(attn_merge<64>, mg, dim3(64), 0, st, a); break;
+    case 96: RF_KLAUNCH(attn_merge<96>, mg, dim3(64), 0, st, a); break;
+    case 128: RF_KLAUNCH(attn_merge<128>, mg, dim3(64), 0, st, a); break;
+    default: RF_KLAUNCH(attn_merge<256>, mg, dim3(64), 0, st, a); break;  // 256 (attention_supported)
+  }
+  return hipGetLastError();
+}
+
+template <int G>
+static void launch_split_g(const AttnArgs& a, uint32_t w, hipStream_t st) {
+  switch (a.hd) {
+    case 64: w == 4 ? launch_split_t<G, 4, 4>(a, st) : launch_split_t<G, 4, 8>(a, st); break;
+    case 96: w == 4 ? launch_split_t<G, 6, 4>(a, st) : launch_split_t<G, 6, 8>(a, st); break;
+    case 128: w == 4 ? launch_split_t<G, 8, 4>(a, st) : launch_split_t<G, 8, 8>(a, st); break;
+    default:
+      if constexpr (G == 1 || G == 2 || G == 4)  // attention_per_kv
+        w == 4 ? launch_split_t<G, 16, 4>(a, st) : launch_split_t<G, 16, 8>(a, st);
+  }
+}
+
 hipError_t launch_attention(const AttnArgs& a, hipStream_t st) {
   if (a.nsplit < 1 || a.nsplit > ATT_MAX_SPLITS) return hipErrorInvalidValue;
   const uint32_t G = a.qh / a.kvh, dpl = a.hd / 16;
   if (a.ntok && !a.per_q && prefill_attention_mfma_supported(a.qh, a.kvh, a.hd, (uint64_t)a.hist + a.ntok)) {
-    switch (G * 1000 + a.hd) {
-      case 1064: launch_apf_t<1, 64>(a, st); break;
-      case 1128: launch_apf_t<1, 128>(a, st); break;
-      case 2064: launch_apf_t<2, 64>(a, st); break;
-      case 2128: launch_apf_t<2, 128>(a, st); break;
-      case 4064: launch_apf_t<4, 64>(a, st); break;
-      case 4128: launch_apf_t<4, 128>(a, st); break;
-      case 8064: launch_apf_t<8, 64>(a, st); break;
-      default: launch_apf_t<8, 128>(a, st); break;
+    switch (G) {
+      case 1: launch_apf_g<1>(a, st); break;
+      case 2: launch_apf_g<2>(a, st); break;
+      case 3: launch_apf_g<3>(a, st); break;
+      case 4: launch_apf_g<4>(a, st); break;
+      case 5: launch_apf_g<5>(a, st); break;
+      case 6: launch_apf_g<6>(a, st); break;
+      case 7: launch_apf_g<7>(a, st); break;
+      default: launch_apf_g<8>(a, st); break;
     }
-    hipError_t e = hipGetLastError();
-    if (e != hipSuccess || a.nsplit == 1 || a.defer_merge) return e;
-    const dim3 mg(a.qh, 1, a.ntok);
-    if (a.hd == 64) RF_KLAUNCH(attn_merge<1>, mg, dim3(64), 0, st, a);
-    else RF_KLAUNCH(attn_merge<2>, mg, dim3(64), 0, st, a);
-    return hipGetLastError();
+    return launch_merge(a, st);
   }
   // API mode knows the context on the host; model mode passes the regime's W.
   const uint32_t w = a.waves ? a.waves : attention_waves(att_chunk(a.hist + 1, a.nsplit), G * a.hd);
   if (w != 4 && w != 8) return hipErrorInvalidValue;
-  bool done = false;
+  if (!attention_supported(a.qh, a.kvh, a.hd, 1) || (!a.per_q && !attention_per_kv(G, a.hd))) return hipErrorInvalidValue;
   if (a.per_q) {  // one workgroup per query head: G = 1 kernels, any GQA ratio
     switch (dpl * 2 + (w == 8 ? 1 : 0)) {
       case 8: launch_split_t<1, 4, 4, true>(a, st); break;
       case 9: launch_split_t<1, 4, 8, true>(a, st); break;
+      case 12: launch_split_t<1, 6, 4, true>(a, st); break;
+      case 13: launch_split_t<1, 6, 8, true>(a, st); break;
       case 16: launch_split_t<1, 8, 4, true>(a, st); break;
       case 17: launch_split_t<1, 8, 8, true>(a, st); break;
       case 32: launch_split_t<1, 16, 4, true>(a, st); break;
-      case 33: launch_split_t<1, 16, 8, true>(a, st); break;
-      default: return hipErrorInvalidValue;
+      default: launch_split_t<1, 16, 8, true>(a, st); break;
     }
-    done = true;
+    return launch_merge(a, st);
   }
-#define RF_ATT(GG, DD)                                          \
-  if (!done && G == GG && dpl == DD) {                          \
-    if (w == 4) launch_split_t<GG, DD, 4>(a, st);               \
-    else launch_split_t<GG, DD, 8>(a, st);                      \
-    done = true;                                                \
+  switch (G) {
+    case 1: launch_split_g<1>(a, w, st); break;
+    case 2: launch_split_g<2>(a, w, st); break;
+    case 3: launch_split_g<3>(a, w, st); break;
+    case 4: launch_split_g<4>(a, w, st); break;
+    case 5: launch_split_g<5>(a, w, st); break;
+    case 6: launch_split_g<6>(a, w, st); break;
+    case 7: launch_split_g<7>(a, w, st); break;
+    default: launch_split_g<8>(a, w, st); break;
   }
-  RF_ATT(1, 4) RF_ATT(1, 8) RF_ATT(1, 16) RF_ATT(2, 4) RF_ATT(2, 8) RF_ATT(2, 16)
-  RF_ATT(4, 4) RF_ATT(4, 8) RF_ATT(4, 16) RF_ATT(8, 4) RF_ATT(8, 8)
-#undef RF_ATT
-  if (!done) return hipErrorInvalidValue;
-  hipError_t e = hipGetLastError();
-  if (e != hipSuccess || a.nsplit == 1 || a.defer_merge) return e;
-  const dim3 mg(a.qh, 1, a.ntok ? a.ntok : 1);
-  switch (a.hd) {
-    case 64: RF_KLAUNCH(attn_merge<1>, mg, dim3(64), 0, st, a); break;
-    case 128: RF_KLAUNCH(attn_merge<2>, mg, dim3(64), 0, st, a); break;
-    default: RF_KLAUNCH(attn_merge<4>, mg, dim3(64), 0, st, a); break;  // 256 (attention_supported)
-  }
-  return hipGetLastError();
+  return launch_merge(a, st);
 }
 
 // Loads this file's code object on the current device (HIP defers that to a
 // kernel's first use, which may otherwise fall inside a stream capture).
 hipError_t load_module_attention() {
   hipFuncAttributes fa;
-  return hipFuncGetAttributes(&fa, reinterpret_cast<const void*>(attn_merge<2>));
+  return hipFuncGetAttributes(&fa, reinterpret_cast<const void*>(attn_merge<128>));
 }
 
 }  // namespace rf

@@ -230,13 +230,16 @@ struct AttnShape {
   uint32_t per_q, nsplit, waves;
 };
 constexpr int ATT_REGIMES = 5;
-int attention_regime(uint64_t total, uint32_t qh, uint32_t kvh, uint64_t cap);
+int attention_regime(uint64_t total, uint32_t qh, uint32_t kvh, uint32_t hd, uint64_t cap);
 void set_attention_single(uint32_t n);
 uint32_t attention_single();
-AttnShape attention_regime_shape(int regime, uint32_t qh, uint32_t kvh, uint64_t cap);
+AttnShape attention_regime_shape(int regime, uint32_t qh, uint32_t kvh, uint32_t hd, uint64_t cap);
 uint64_t attention_ws_floats(uint32_t nsplit, uint32_t qh, uint32_t hd);
 // The split kernel handles this shape for up to `total_positions` positions.
 bool attention_supported(uint32_t qh, uint32_t kvh, uint32_t hd, uint64_t total_positions);
+// It has a form with the G = qh / kvh query heads of a KV head in one
+// workgroup (else its launches are per query head, per_q).
+bool attention_per_kv(uint32_t G, uint32_t hd);
 
 // Batched prefill (rf_prefill.hip): Y[t][r] = sum_k W[r][k] X[t][k] for up to
 // MM_MAX_TOKENS tokens on the packed layout, on the matrix cores, with split-K

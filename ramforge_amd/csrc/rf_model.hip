@@ -1374,7 +1374,8 @@ int32_t enqueue_qkv(rf_model* m, size_t li) {
 // a single shape.
 int attn_regime(const rf_model* m, uint64_t pos) {
   if (!m->attn_fast) return 0;
-  return attention_regime(pos + 1, (uint32_t)m->cfg.head_count, (uint32_t)m->cfg.head_count_kv, m->kv_max);
+  return attention_regime(pos + 1, (uint32_t)m->cfg.head_count, (uint32_t)m->cfg.head_count_kv,
+                          (uint32_t)m->cfg.head_dim, m->kv_max);
 }
 
 // Whether layer li's o-projection merges the attention's chunk records
@@ -1408,7 +1409,7 @@ int32_t enqueue_attention(rf_model* m, size_t li) {
   a.ws = m->attn_ws; a.rope = m->rope; a.k_store = kc; a.v_store = vc; a.d_pos = m->d_pos;
   a.qh = (uint32_t)c.head_count; a.kvh = (uint32_t)c.head_count_kv; a.hd = (uint32_t)hd;
   // the position this step processes picks the shape
-  const AttnShape sh = attention_regime_shape(attn_regime(m, m->seq_len), a.qh, a.kvh, m->kv_max);
+  const AttnShape sh = attention_regime_shape(attn_regime(m, m->seq_len), a.qh, a.kvh, a.hd, m->kv_max);
   a.per_q = sh.per_q; a.nsplit = sh.nsplit; a.waves = sh.waves;
   m->oproj_merge = false;
   bool merge = false;
@@ -1429,7 +1430,7 @@ int32_t enqueue_oproj(rf_model* m, size_t li) {
   if (m->oproj_merge) {  // the attention just enqueued left its chunk records
     m->oproj_merge = false;
     const AttnShape sh = attention_regime_shape(attn_regime(m, m->seq_len), (uint32_t)c.head_count,
-                                                (uint32_t)c.head_count_kv, m->kv_max);
+                                                (uint32_t)c.head_count_kv, (uint32_t)c.head_dim, m->kv_max);
     const PkMerge mg{m->attn_ws, m->d_pos, sh.nsplit, (uint32_t)c.head_count, (uint32_t)c.head_dim};
     PkSegDesc ps{L.o.d, nullptr, L.o.ne1, 0, d, m->hidden, m->hidden};
     RF_LAUNCH(launch_matvec_packed(L.o.type, &ps, 1, m->attn_out, nullptr, 0.f, qd, EPI_RESIDUAL, m->ctx->compute,
@@ -1860,7 +1861,7 @@ int32_t enqueue_prefill_layer(rf_model* m, size_t li, uint64_t pos0, uint64_t nt
     // workgroups, one per KV head (its query heads share each K/V row read)
     // and chunks of up to ATT_MAX_CHUNK positions, so up to 1024 positions
     // need no merge.
-    a.per_q = 0;
+    a.per_q = attention_per_kv(a.qh / a.kvh, a.hd) ? 0 : 1;
     a.nsplit = prefill_attention_mfma_supported(a.qh, a.kvh, a.hd, pos0 + nt)
                    ? prefill_attention_mfma_splits(pos0 + nt, nt, a.kvh)
                    : prefill_attn_splits(pos0 + nt);
@@ -2035,7 +2036,8 @@ int32_t model_create(rf_ctx* ctx, const rf_model_config* cfg, uint64_t kv_cap, u
   m->attn_fast = fast;
   m->attn_chunks = 1;
   for (int r = 0; fast && r < ATT_REGIMES; ++r) {
-    const AttnShape sh = attention_regime_shape(r, (uint32_t)c.head_count, (uint32_t)c.head_count_kv, kv_cap);
+    const AttnShape sh = attention_regime_shape(r, (uint32_t)c.head_count, (uint32_t)c.head_count_kv,
+                                                (uint32_t)c.head_dim, kv_cap);
     if (sh.nsplit > m->attn_chunks) m->attn_chunks = sh.nsplit;
   }
   const uint64_t ws_floats = fast ? attention_ws_floats(m->attn_chunks, (uint32_t)c.head_count, (uint32_t)c.head_dim)

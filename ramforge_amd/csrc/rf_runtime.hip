@@ -1057,7 +1057,7 @@ int32_t attention_setup(const float* q, const float* kh, const float* vh, const 
   *fast = attention_supported(qh, kvh, hd, total) && aligned(q) && (hist == 0 || (aligned(kh) && aligned(vh))) &&
           aligned(kc) && aligned(vc);
   if (*fast) {  // the context is known here: its own regime, sized to itself
-    const AttnShape sh = attention_regime_shape(attention_regime(total, qh, kvh, total), qh, kvh, total);
+    const AttnShape sh = attention_regime_shape(attention_regime(total, qh, kvh, hd, total), qh, kvh, hd, total);
     a->per_q = sh.per_q; a->nsplit = sh.nsplit; a->waves = sh.waves;
     *ws_bytes = attention_ws_floats(a->nsplit, qh, hd) * 4;
   } else {
@@ -1118,7 +1118,7 @@ uint64_t rf_attention_workspace_bytes(uint64_t max_positions, uint32_t qh, uint3
   const uint32_t total = (uint32_t)max_positions;
   uint32_t nsplit = 1;
   for (int r = 0; r < ATT_REGIMES; ++r)
-    nsplit = std::max(nsplit, attention_regime_shape(r, qh, kvh, total).nsplit);
+    nsplit = std::max(nsplit, attention_regime_shape(r, qh, kvh, hd, total).nsplit);
   const uint64_t split = attention_ws_floats(nsplit, qh, hd) * 4;
   const uint64_t naive = (uint64_t)qh * max_positions * 4;
   return std::max(split, naive);

@@ -397,7 +397,9 @@ int32_t rf_model_decode_steps(rf_model *model, uint64_t steps);
 /* Copies the last `n` greedy tokens produced by rf_model_decode_steps. */
 int32_t rf_model_read_tokens(rf_model *model, uint32_t *out, uint64_t n);
 /* Batched prompt prefill: forwards tokens[0..n) at positions seq_len ..
- * seq_len + n - 1 in chunks of 64 tokens, each chunk through every layer
+ * seq_len + n - 1 in chunks of up to 512 tokens (64 where the VRAM budget
+ * refuses the longer chunks' workspace, single forwards where it refuses
+ * those too), each chunk through every layer
  * with the projections as rf_matmul_packed GEMMs, per-token RMSNorm, RoPE,
  * K/V cache writes and causal attention over the cache.  Same result as n
  * rf_model_forward calls (the reference's prompt loop, inference.rs:580-592)

@@ -1082,8 +1082,9 @@ template <int G> constexpr int apf_tiles() { return G <= 4 ? 2 : 1; }
 uint32_t prefill_attention_mfma_splits(uint64_t total, uint64_t ntok, uint32_t kvh) {
   const uint64_t per = APF_TOK * 2;  // workgroups of two token tiles (G > 4: one; more splits then)
   const uint64_t tiles = (ntok + per - 1) / per * (kvh ? kvh : 1);
-  uint64_t n = (256 + tiles - 1) / tiles;
-  const uint64_t by_len = (total + 255) / 256, most = (total + ATT_MIN_CHUNK - 1) / ATT_MIN_CHUNK;
+  // chunks of more than two workgroup tiles bring the workgroups themselves
+  uint64_t n = ntok > 2 * per ? (512 + tiles - 1) / tiles : (256 + tiles - 1) / tiles;
+  const uint64_t by_len = ntok > 2 * per ? 1 : (total + 255) / 256, most = (total + ATT_MIN_CHUNK - 1) / ATT_MIN_CHUNK;
   if (n < by_len) n = by_len;
   if (n > 32) n = 32;
   if (n > most) n = most;

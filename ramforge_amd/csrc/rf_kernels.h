@@ -245,7 +245,8 @@ bool attention_per_kv(uint32_t G, uint32_t hd);
 // MM_MAX_TOKENS tokens on the packed layout, on the matrix cores, with split-K
 // partials in `part` and the epilogue of the decode matvec (EPI_SWIGLU:
 // segment 0 gate, segment 1 up, output in segment 0's y).
-constexpr uint64_t MM_MAX_TOKENS = 64;
+constexpr uint64_t MM_MAX_TOKENS = 512;
+constexpr uint64_t MM_SMALL_TOKENS = 64;  // up to here mm_packed (rf_prefill.hip), beyond the tiled kernel (rf_gemm.hip)
 struct MmSegDesc {
   const void* packed;    // packed matrix base
   uint64_t matrix_rows;  // rows of the whole packed matrix (locates its regions)

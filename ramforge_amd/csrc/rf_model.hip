@@ -132,6 +132,7 @@ struct rf_model {
   std::vector<LayerRes> res;
   // Batched prefill (rf_model_prefill): activations of one chunk of prompt
   // tokens and its workspaces, charged "tmp:prefill" at the first use.
+  uint64_t p_chunk = 0;  // tokens of one chunk
   bool prefill_batched = false;  // rf_model_generate forwards its prompt batched
   float *p_h = nullptr, *p_xn = nullptr, *p_q = nullptr, *p_k = nullptr, *p_v = nullptr, *p_qr = nullptr;
   float *p_a = nullptr, *p_act = nullptr, *p_up = nullptr, *p_part = nullptr, *p_att = nullptr;
@@ -1709,7 +1710,7 @@ int32_t forward_token(rf_model* m, uint32_t token, uint64_t pos) {
 }
 
 // ---------------------------------------------------------------- prefill
-// A chunk of up to MM_MAX_TOKENS prompt tokens through one layer
+// A chunk of up to p_chunk prompt tokens through one layer
 // (model_executor.rs:102-236 for each token): the projections as GEMMs over
 // the chunk (rf_prefill.hip), RMSNorm per token, RoPE + K/V cache rows, then
 // causal attention of each token over the cache up to its own position.
@@ -1731,10 +1732,10 @@ bool prefill_supported(const rf_model* m) {
   return true;
 }
 
-int32_t ensure_prefill_ws(rf_model* m) {
-  if (m->p_h) return RF_OK;
+// The prefill workspace for chunks of up to T tokens.
+int32_t alloc_prefill_ws(rf_model* m, uint64_t T) {
   const rf_model_config& c = m->cfg;
-  const uint64_t T = MM_MAX_TOKENS, d = c.embedding_length, hd = c.head_dim, qd = c.head_count * hd;
+  const uint64_t d = c.embedding_length, hd = c.head_dim, qd = c.head_count * hd;
   const uint64_t kvd = c.head_count_kv * hd, f = c.feed_forward_length;
   // split-K partials: the largest of the launches a layer makes
   uint64_t part = 0;
@@ -1784,7 +1785,18 @@ int32_t ensure_prefill_ws(rf_model* m) {
   }
   m->p_tok = reinterpret_cast<uint32_t*>(base);
   m->p_part_floats = part;
+  m->p_chunk = T;
   return RF_OK;
+}
+
+// Chunks of MM_MAX_TOKENS tokens (fewer where the cache never holds as many),
+// or of MM_SMALL_TOKENS where the budget refuses their workspace.
+int32_t ensure_prefill_ws(rf_model* m) {
+  if (m->p_h) return RF_OK;
+  const uint64_t T = std::min<uint64_t>(MM_MAX_TOKENS, std::max<uint64_t>(MM_SMALL_TOKENS, (m->kv_max + 31) / 32 * 32));
+  int32_t rc = alloc_prefill_ws(m, T);
+  if (rc == RF_ERR_BUDGET && T > MM_SMALL_TOKENS) rc = alloc_prefill_ws(m, MM_SMALL_TOKENS);
+  return rc;
 }
 
 // A streaming model gives the prefill workspace back after the prompt: its
@@ -1903,19 +1915,20 @@ int32_t prefill_tokens(rf_model* m, const uint32_t* tokens, uint64_t n) {
   int32_t rc = check_ready(m);
   if (rc) return rc;
   if ((rc = ensure_kv(m, m->seq_len + n))) return rc;
-  if (!prefill_supported(m)) {
+  const bool batched = prefill_supported(m);
+  if (batched && (rc = ensure_prefill_ws(m)) && rc != RF_ERR_BUDGET) return rc;
+  if (!batched || rc) {  // unsupported, or a budget without room for the workspace
     for (uint64_t i = 0; i < n; ++i)
       if ((rc = forward_token(m, tokens[i], m->seq_len))) return rc;
     return RF_OK;
   }
-  if ((rc = ensure_prefill_ws(m))) return rc;
   const rf_model_config& c = m->cfg;
   hipStream_t st = m->ctx->compute;
   const uint64_t d = c.embedding_length;
   const uint32_t nl = (uint32_t)m->layers.size();
   uint64_t nt = 0;
   for (uint64_t off = 0; off < n; off += nt) {
-    nt = n - off < MM_MAX_TOKENS ? n - off : MM_MAX_TOKENS;
+    nt = n - off < m->p_chunk ? n - off : m->p_chunk;
     const uint64_t pos0 = m->seq_len;
     RF_LAUNCH(hipMemcpyAsync(m->p_tok, tokens + off, nt * 4, hipMemcpyHostToDevice, st), "upload prompt tokens");
     RF_LAUNCH(launch_dequant_rows(m->token_embd.type, m->token_embd.d, d, nt, m->p_h, m->p_tok, c.vocab_size, st),

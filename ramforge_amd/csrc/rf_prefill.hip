@@ -6,7 +6,11 @@
 // ModelExecutor::execute_layer per token, model_executor.rs:102-236); this
 // file computes the same per-token arithmetic for up to MM_MAX_TOKENS tokens
 // per launch, so each weight byte is read once per chunk instead of once per
-// token.
+// token.  Launches of more than MM_SMALL_TOKENS tokens run the tiled GEMM of
+// rf_gemm.hip: it decodes the weights and splits x once for all the tokens
+// (Q8_0, 512 tokens: 28672 x 4096 562 us in eight mm_packed launches against
+// 415, 4096 x 14336 322 against 210, 4096 x 4096 168 against 74; at 65 to 128
+// tokens the two meet, 36 against 35 us for 4096 x 4096 and 96 tokens).
 //
 // GEMM (mm_packed): Y[t][r] = sum_k W[r][k] X[t][k] on the packed layout of
 // Q8_0 / Q4_0 / Q4_K / Q6_K (rf_matvec_packed.hip).  Per 32-element step the
@@ -43,6 +47,7 @@
 #include <algorithm>
 
 #include "rf_device.h"
+#include "rf_gemm.h"
 #include "rf_kernels.h"
 
 namespace rf {
@@ -796,13 +801,17 @@ static void mm_shape(uint64_t groups, uint64_t in_dim, uint64_t n, uint32_t* nsp
   *nslices = (uint32_t)ns;
 }
 
+static bool mm_tiled(uint64_t n) { return n > MM_SMALL_TOKENS; }
+
 static uint64_t mm_groups(const MmSegDesc* segs, int nseg, uint64_t rows_per_group) {
   uint64_t g = 0;
   for (int i = 0; i < nseg; ++i) g += (segs[i].rows + rows_per_group - 1) / rows_per_group;
   return g;
 }
 
-// Partial-sum floats of a launch of exactly n tokens, for either workgroup size.
+// Workspace floats of a launch of exactly n tokens: the tiled kernel's x
+// planes and partial sums, or mm_packed's partial sums for either workgroup
+// size.
 uint64_t mm_part_floats_at(const uint64_t* rows, int nseg, uint64_t in_dim, uint64_t n) {
   MmSegDesc d[3] = {};
   uint64_t mtot = 0;
@@ -810,6 +819,7 @@ uint64_t mm_part_floats_at(const uint64_t* rows, int nseg, uint64_t in_dim, uint
     d[i].rows = rows[i];
     mtot += rows[i];
   }
+  if (mm_tiled(n)) return mm_tile_ws_floats(mm_groups(d, nseg, MM_TILE_ROWS), mtot, in_dim, n);
   uint64_t most = 0;
   for (uint64_t rpg : {MM_ROWS_NARROW, MM_ROWS_WIDE}) {
     uint32_t nsplit, spp, ns;
@@ -819,12 +829,12 @@ uint64_t mm_part_floats_at(const uint64_t* rows, int nseg, uint64_t in_dim, uint
   return most * mtot;
 }
 
-// Partial-sum floats a launch of up to n tokens may need, for either
-// workgroup size (the split count depends on the token count and on the
-// workgroups a launch has).
+// Workspace floats a launch of up to n tokens may need (the split count
+// depends on the token count; the tiled kernel's only on the 32-token tiles).
 uint64_t mm_part_floats(const uint64_t* rows, int nseg, uint64_t in_dim, uint64_t n) {
   uint64_t most = 0;
-  for (uint64_t k = 1; k <= n; ++k) most = std::max(most, mm_part_floats_at(rows, nseg, in_dim, k));
+  for (uint64_t k = 1; k <= n; k = mm_tiled(k + 1) && k < n ? std::min(n, (k / 32 + 1) * 32) : k + 1)
+    most = std::max(most, mm_part_floats_at(rows, nseg, in_dim, k));
   return most;
 }
 
@@ -906,7 +916,8 @@ hipError_t launch_matmul_packed(uint32_t t, const MmSegDesc* segs, int nseg, con
       return hipErrorInvalidValue;
   }
   if (!mm_supported(t, in_dim) || nseg < 1 || nseg > 3 || n == 0 || n > MM_MAX_TOKENS) return hipErrorInvalidValue;
-  if (!al16(x) || ldx % 4 != 0 || ldx < in_dim || !part) return hipErrorInvalidValue;
+  const bool tiled = mm_tiled(n);
+  if ((!tiled && (!al16(x) || ldx % 4 != 0)) || ldx < in_dim || !part) return hipErrorInvalidValue;
   if (epi == EPI_SWIGLU && (nseg != 2 || segs[0].rows != segs[1].rows)) return hipErrorInvalidValue;
   const int nreg = t == T_Q6_K ? 4 : 2;
   auto row_bytes = [&](int k) -> uint64_t { return mm_row_bytes(t, k, in_dim); };
@@ -914,6 +925,7 @@ hipError_t launch_matmul_packed(uint32_t t, const MmSegDesc* segs, int nseg, con
   // offsets, with offsets from MM_OOR on reading as zeros
   if ((uint64_t)n * ldx * 4 >= (1ull << 31)) return hipErrorInvalidValue;
   bool sc8 = in_dim % MM_KS == 0;
+  MmTileSeg ts[3] = {};
   const bool wide = mm_pick_wide(t, segs, nseg, in_dim, n);
   const uint64_t rpg = wide ? MM_ROWS_WIDE : MM_ROWS_NARROW;
   MmArgs a{};
@@ -928,8 +940,12 @@ hipError_t launch_matmul_packed(uint32_t t, const MmSegDesc* segs, int nseg, con
       a.seg[i].reg[k] = static_cast<const uint8_t*>(d.packed) + off + d.row_start * rb;
       off += d.matrix_rows * rb;
     }
-    for (int k = 0; k < nreg; ++k)
+    for (int k = 0; k < nreg; ++k) {
       if (d.rows * row_bytes(k) >= (1ull << 31)) return hipErrorInvalidValue;
+      ts[i].reg[k] = a.seg[i].reg[k];
+      ts[i].bytes[k] = d.rows * row_bytes(k);
+    }
+    ts[i].rows = d.rows;
     sc8 = sc8 && (reinterpret_cast<uintptr_t>(a.seg[i].reg[1]) & 7u) == 0;
     // 8-byte code loads; Q4_K headers and Q6_K scales as 16 bytes
     if ((reinterpret_cast<uintptr_t>(a.seg[i].reg[0]) & 7u) != 0) return hipErrorInvalidValue;
@@ -945,9 +961,11 @@ hipError_t launch_matmul_packed(uint32_t t, const MmSegDesc* segs, int nseg, con
     mtot += d.rows;
   }
   if (mtot > 0xFFFFFFFFull || groups > 0x7FFFFFFFull) return hipErrorInvalidValue;
-  uint32_t nsplit, spp, nslices;
-  mm_shape(groups, in_dim, n, &nsplit, &spp, &nslices);
-  if ((uint64_t)nsplit * n * mtot > part_floats) return hipErrorInvalidValue;
+  uint32_t nsplit = 1, spp = 1, nslices = 1;
+  if (!tiled) {
+    mm_shape(groups, in_dim, n, &nsplit, &spp, &nslices);
+    if ((uint64_t)nsplit * n * mtot > part_floats) return hipErrorInvalidValue;
+  }
   a.nseg = (uint32_t)nseg;
   a.x = x;
   a.part = part;
@@ -968,11 +986,18 @@ hipError_t launch_matmul_packed(uint32_t t, const MmSegDesc* segs, int nseg, con
   r.part = part;
   if (rope && !mm_reduce_vec4(r)) return hipErrorInvalidValue;  // before any launch
   hipError_t e;
-  switch (t) {
-    case T_Q8_0: e = mm_launch_shape<T_Q8_0>(a, grid, ntt, wide, sc8, st); break;
-    case T_Q4_0: e = mm_launch_shape<T_Q4_0>(a, grid, ntt, wide, sc8, st); break;
-    case T_Q4_K: e = mm_launch_shape<T_Q4_K>(a, grid, ntt, wide, false, st); break;
-    default: e = mm_launch_shape<T_Q6_K>(a, grid, ntt, wide, false, st); break;
+  if (tiled) {
+    MmTileOut o{};
+    e = launch_mm_tile(t, ts, nseg, x, ldx, n, in_dim, part, part_floats, st, &o);
+    r.part = o.part;
+    r.nsplit = o.nsplit;
+  } else {
+    switch (t) {
+      case T_Q8_0: e = mm_launch_shape<T_Q8_0>(a, grid, ntt, wide, sc8, st); break;
+      case T_Q4_0: e = mm_launch_shape<T_Q4_0>(a, grid, ntt, wide, sc8, st); break;
+      case T_Q4_K: e = mm_launch_shape<T_Q4_K>(a, grid, ntt, wide, false, st); break;
+      default: e = mm_launch_shape<T_Q6_K>(a, grid, ntt, wide, false, st); break;
+    }
   }
   if (e != hipSuccess) return e;
   const uint64_t total = (uint64_t)n * r.mcols;
@@ -1103,7 +1128,8 @@ hipError_t launch_rope_kv_rows(const float* q, const float* k, const float* v, c
 hipError_t load_module_prefill() {
   (void)mm_cu_count();
   hipFuncAttributes fa;
-  return hipFuncGetAttributes(&fa, reinterpret_cast<const void*>(mm_reduce));
+  const hipError_t e = load_module_gemm();
+  return e != hipSuccess ? e : hipFuncGetAttributes(&fa, reinterpret_cast<const void*>(mm_reduce));
 }
 
 }  // namespace rf

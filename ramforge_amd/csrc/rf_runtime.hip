@@ -946,13 +946,17 @@ int32_t rf_matvec_packed(rf_ctx* ctx, uint32_t t, const void* packed, uint64_t p
   return launch_packed_rows(ctx, t, packed, out_dim, in_dim, x, y, row_start, count, pick_stream(ctx, s));
 }
 
-uint64_t rf_matmul_workspace_bytes(uint64_t out_dim, uint64_t in_dim, uint64_t n_tokens) {
-  if (out_dim == 0 || in_dim == 0 || n_tokens == 0) return 0;
-  const uint64_t chunk = n_tokens < MM_MAX_TOKENS ? n_tokens : MM_MAX_TOKENS;
-  // the launches are chunk tokens each, the last one the remainder
+// Workspace bytes of a matmul in launches of `chunk` tokens, the last one the remainder.
+static uint64_t matmul_ws_bytes(uint64_t out_dim, uint64_t in_dim, uint64_t n_tokens, uint64_t chunk) {
+  if (n_tokens < chunk) chunk = n_tokens;
   uint64_t part = mm_part_floats_at(&out_dim, 1, in_dim, chunk);
   if (n_tokens % chunk) part = std::max(part, mm_part_floats_at(&out_dim, 1, in_dim, n_tokens % chunk));
   return part * 4;
+}
+
+uint64_t rf_matmul_workspace_bytes(uint64_t out_dim, uint64_t in_dim, uint64_t n_tokens) {
+  if (out_dim == 0 || in_dim == 0 || n_tokens == 0) return 0;
+  return matmul_ws_bytes(out_dim, in_dim, n_tokens, MM_MAX_TOKENS);
 }
 
 int32_t rf_matmul_packed(rf_ctx* ctx, uint32_t t, const void* packed, uint64_t packed_bytes, uint64_t out_dim,
@@ -981,19 +985,27 @@ int32_t rf_matmul_packed(rf_ctx* ctx, uint32_t t, const void* packed, uint64_t p
     return set_error(RF_ERR_UNSUPPORTED, "packed %s matmul does not cover %llu x %llu", nm,
                      (unsigned long long)out_dim, (unsigned long long)in_dim);
   hipStream_t st = pick_stream(ctx, s);
-  const uint64_t chunk = n_tokens < MM_MAX_TOKENS ? n_tokens : MM_MAX_TOKENS;
-  int32_t rc = ensure_workspace(ctx, ctx->mm_ws, "workspace:matmul", rf_matmul_workspace_bytes(out_dim, in_dim, n_tokens),
-                                st);
+  // A workspace that cannot grow to the long chunks' size (fixed, being
+  // captured, over the budget) may still hold the short ones'.
+  uint64_t chunk = MM_MAX_TOKENS;
+  int32_t rc = ensure_workspace(ctx, ctx->mm_ws, "workspace:matmul", matmul_ws_bytes(out_dim, in_dim, n_tokens, chunk), st);
+  if ((rc == RF_ERR_INVALID || rc == RF_ERR_BUDGET) && n_tokens > MM_SMALL_TOKENS) {
+    chunk = MM_SMALL_TOKENS;
+    rc = ensure_workspace(ctx, ctx->mm_ws, "workspace:matmul", matmul_ws_bytes(out_dim, in_dim, n_tokens, chunk), st);
+  }
   if (rc) return rc;
+  // launches of up to MM_SMALL_TOKENS tokens stage x with 16-byte loads
   const bool aligned = (reinterpret_cast<uintptr_t>(x) & 15u) == 0 && in_dim % 4 == 0;
-  if (!aligned) {  // the kernel stages x with 16-byte loads
-    rc = ensure_workspace(ctx, ctx->scratch_ws, "workspace:scratch", chunk * in_dim * 4, st);
+  const uint64_t last = n_tokens % chunk ? n_tokens % chunk : chunk, small = chunk <= MM_SMALL_TOKENS ? std::min(chunk, n_tokens)
+                        : last <= MM_SMALL_TOKENS ? last : 0;
+  if (!aligned && small) {
+    rc = ensure_workspace(ctx, ctx->scratch_ws, "workspace:scratch", small * in_dim * 4, st);
     if (rc) return rc;
   }
-  for (uint64_t off = 0; off < n_tokens; off += MM_MAX_TOKENS) {
-    const uint64_t nt = n_tokens - off < MM_MAX_TOKENS ? n_tokens - off : MM_MAX_TOKENS;
+  for (uint64_t off = 0; off < n_tokens; off += chunk) {
+    const uint64_t nt = n_tokens - off < chunk ? n_tokens - off : chunk;
     const float* xc = x + off * in_dim;
-    if (!aligned) {
+    if (!aligned && nt <= MM_SMALL_TOKENS) {
       RF_HIP(hipMemcpyAsync(ctx->scratch_ws.ptr, xc, nt * in_dim * 4, hipMemcpyDeviceToDevice, st), "hipMemcpyAsync");
       xc = static_cast<const float*>(ctx->scratch_ws.ptr);
     }

@@ -149,6 +149,11 @@ PkPlan plan_packed(uint32_t t, uint64_t in_dim);
 hipError_t launch_matvec_packed(uint32_t t, const PkSegDesc* segs, int nseg, const float* x, const float* norm_w,
                                 float eps, uint64_t in_dim, int epi, hipStream_t st, int32_t* advance = nullptr,
                                 const PkMerge* mrg = nullptr);
+// The same kernels on GGUF bytes (any alignment): Q8_0, Q4_0, Q5_0, Q4_K,
+// Q5_K, Q6_K rows of a plain y = W x with a 16-byte aligned x.
+PkPlan plan_gguf(uint32_t t, uint64_t in_dim);
+hipError_t launch_matvec_gguf(uint32_t t, const void* w, uint64_t rows, const float* x, float* y, uint64_t in_dim,
+                              const PkPlan& p, hipStream_t st);
 // hipSuccess when launch_matvec_packed can merge attention chunk records into
 // x for this projection (EPI_RESIDUAL, no norm, one segment of `rows` rows):
 // the single-step launch of Q8_0 / Q4_0 / Q4_K with in_dim = qh * hd, hd a

@@ -62,6 +62,7 @@ typedef __amdgpu_buffer_rsrc_t PkRsrc;
 //   NREG         regions; row_bytes(k, in) = bytes of region k per row
 //   Meta         what a lane loads besides its 16 code bytes
 //   fetch        loads of one lane at code byte b of the row
+//   code         the lane's code word i (0 .. 3)
 //   unit_elem    first element of unit h of the lane whose codes start at b
 //   word         decode code word i against x words (units 0 and 1)
 //   finish       scale the unit sums into the chunk's contribution
@@ -108,6 +109,7 @@ template <> struct PkFmt<T_Q8_0> {
     q = __builtin_amdgcn_raw_buffer_load_b128(r[0], b, 0, PK_AUX_NT);
     m = __builtin_amdgcn_raw_buffer_load_b16(r[1], (b >> 5) << 1, 0, 0);  // block b/32, 2 bytes each
   }
+  __device__ static uint32_t code(const Lane&, const nv_u32x4& q, const Meta&, int i) { return q[i]; }
   __device__ static uint32_t unit_elem(uint32_t b, uint32_t) { return b; }
   // signed codes times x, each product exact up to its own rounding (a zero
   // code adds exactly nothing, as the reference's (q * d) * x does)
@@ -116,7 +118,7 @@ template <> struct PkFmt<T_Q8_0> {
     s0 = fmaf(rf_sb(q, 0), xv.x, s0); s0 = fmaf(rf_sb(q, 1), xv.y, s0);
     s0 = fmaf(rf_sb(q, 2), xv.z, s0); s0 = fmaf(rf_sb(q, 3), xv.w, s0);
   }
-  __device__ static float finish(const Lane&, const Meta& m, float s0, float, float, float) {
+  __device__ static float finish(const Lane&, const nv_u32x4&, const Meta& m, float s0, float, float, float) {
     return rf_half_to_float_fast(m) * s0;
   }
   // the codes are signed bytes: one dot4 per word and digit plane
@@ -152,6 +154,8 @@ template <> struct PkFmt<T_Q4_0> {
     q = __builtin_amdgcn_raw_buffer_load_b128(r[0], b, 0, PK_AUX_NT);
     m = __builtin_amdgcn_raw_buffer_load_b16(r[1], (b >> 4) << 1, 0, 0);  // block b/16
   }
+  template <class M>
+  __device__ static uint32_t code(const Lane&, const nv_u32x4& q, const M&, int i) { return q[i]; }
   // byte j: low nibble -> element j, high nibble -> element j + 16 (quant.rs:84-113)
   __device__ static uint32_t unit_elem(uint32_t b, uint32_t h) { return 2u * b + 16u * h; }
   // The signed codes nibble - 8 as int8 bytes 16 (nibble - 8): products with
@@ -168,7 +172,7 @@ template <> struct PkFmt<T_Q4_0> {
     s1 = fmaf(rf_sb(hi, 0), xw.x, s1); s1 = fmaf(rf_sb(hi, 1), xw.y, s1);
     s1 = fmaf(rf_sb(hi, 2), xw.z, s1); s1 = fmaf(rf_sb(hi, 3), xw.w, s1);
   }
-  __device__ static float finish(const Lane&, const Meta& m, float s0, float s1, float, float) {
+  __device__ static float finish(const Lane&, const nv_u32x4&, const Meta& m, float s0, float s1, float, float) {
     return rf_half_to_float_fast(m) * ((s0 + s1) * 0.0625f);
   }
   // the same int8 bytes 16 (nibble - 8) against the digits: exact int32 sums
@@ -223,6 +227,8 @@ template <> struct PkFmt<T_Q4_K> {
     q = __builtin_amdgcn_raw_buffer_load_b128(r[0], b, 0, PK_AUX_NT);
     m = __builtin_amdgcn_raw_buffer_load_b128(r[1], (b >> 7) << 4, 0, 0);
   }
+  template <class M>
+  __device__ static uint32_t code(const Lane&, const nv_u32x4& q, const M&, int i) { return q[i]; }
   __device__ static uint32_t unit_elem(uint32_t b, uint32_t h) {
     const uint32_t o = b & 127u;
     return (b >> 7) * 256u + 64u * (o >> 5) + 16u * ((o >> 4) & 1u) + 32u * h;
@@ -236,7 +242,7 @@ template <> struct PkFmt<T_Q4_K> {
     s1 = fmaf(rf_ub(hi, 0), xw.x, s1); s1 = fmaf(rf_ub(hi, 1), xw.y, s1);
     s1 = fmaf(rf_ub(hi, 2), xw.z, s1); s1 = fmaf(rf_ub(hi, 3), xw.w, s1);
   }
-  __device__ static float finish(const Lane& L, const Meta& m, float s0, float s1, float xs0, float xs1) {
+  __device__ static float finish(const Lane& L, const nv_u32x4&, const Meta& m, float s0, float s1, float xs0, float xs1) {
     // sub-blocks j = 2g (+0) and 2g + 1 (+8 bits): for j < 4 sc = S[j] & 63,
     // m = S[j+4] & 63; else sc = (S[j+4] & 15) | (S[j-4] >> 6) << 4,
     // m = (S[j+4] >> 4) | (S[j] >> 6) << 4  (S = the 12 scale bytes)
@@ -252,18 +258,21 @@ template <> struct PkFmt<T_Q4_K> {
     const float r0 = fmaf(d * (float)sc[0], s0, -(dmin * (float)mn[0]) * xs0);
     return fmaf(d * (float)sc[1], s1, fmaf(-(dmin * (float)mn[1]), xs1, r0));
   }
+  // d * sc and dmin * m of sub-block 2g + h
+  __device__ static void scale_min(const Lane& L, const Meta& m, int h, float& d1, float& m1) {
+    const float d = rf_half_to_float_fast(m.x & 0xFFFFu), dmin = rf_half_to_float_fast(m.x >> 16);
+    const uint32_t s = L.sh + 8u * h;
+    const uint32_t a = (m.y >> s) & 0xFFu, c = (m.z >> s) & 0xFFu, e = (m.w >> s) & 0xFFu;
+    d1 = d * (float)(L.hi ? ((e & 15u) | ((a >> 6) << 4)) : (a & 63u));
+    m1 = dmin * (float)(L.hi ? ((e >> 4) | ((c >> 6) << 4)) : (c & 63u));
+  }
   // d1 * q - m1 with d1 = d * sc, m1 = dmin * m (quant.rs:228-254), no fused multiply-add
   __device__ static uint32_t kinds(const Lane& L, uint32_t q, const Meta& m, int, const float4& xv, const float4& xw) {
-    const float d = rf_half_to_float_fast(m.x & 0xFFFFu), dmin = rf_half_to_float_fast(m.x >> 16);
     uint32_t out = 0;
 #pragma unroll
     for (int h = 0; h < 2; ++h) {
-      const uint32_t s = L.sh + 8u * h;
-      const uint32_t a = (m.y >> s) & 0xFFu, c = (m.z >> s) & 0xFFu, e = (m.w >> s) & 0xFFu;
-      const uint32_t sc = L.hi ? ((e & 15u) | ((a >> 6) << 4)) : (a & 63u);
-      const uint32_t mn = L.hi ? ((e >> 4) | ((c >> 6) << 4)) : (c & 63u);
-      const float d1 = d * (float)sc, m1 = dmin * (float)mn;
-      float deq[4];
+      float d1, m1, deq[4];
+      scale_min(L, m, h, d1, m1);
 #pragma unroll
       for (int k = 0; k < 4; ++k) {
         const float prod = d1 * (float)((q >> (8 * k + 4 * h)) & 0xFu);
@@ -307,6 +316,7 @@ template <> struct PkFmt<T_Q6_K> {
     m.sc = __builtin_amdgcn_raw_buffer_load_b128(r[2], blk * 16u, 0, 0);
     m.d = __builtin_amdgcn_raw_buffer_load_b16(r[3], blk * 2u, 0, 0);
   }
+  __device__ static uint32_t code(const Lane&, const nv_u32x4& q, const Meta&, int i) { return q[i]; }
   __device__ static uint32_t unit_elem(uint32_t b, uint32_t h) {
     const uint32_t o = b & 127u;
     return (b >> 7) * 256u + 128u * (o >> 6) + (o & 63u) + 64u * h;
@@ -324,7 +334,7 @@ template <> struct PkFmt<T_Q6_K> {
     s1 = fmaf(rf_sb(hi, 0), xw.x, s1); s1 = fmaf(rf_sb(hi, 1), xw.y, s1);
     s1 = fmaf(rf_sb(hi, 2), xw.z, s1); s1 = fmaf(rf_sb(hi, 3), xw.w, s1);
   }
-  __device__ static float finish(const Lane& L, const Meta& m, float s0, float s1, float, float) {
+  __device__ static float finish(const Lane& L, const nv_u32x4&, const Meta& m, float s0, float s1, float, float) {
     const uint32_t w0 = L.hf ? m.sc.z : m.sc.x, w1 = L.hf ? m.sc.w : m.sc.y;
     const float sc0 = (float)(int32_t)(int8_t)((w0 >> L.bsh) & 0xFFu);
     const float sc1 = (float)(int32_t)(int8_t)((w1 >> L.bsh) & 0xFFu);
@@ -349,6 +359,244 @@ template <> struct PkFmt<T_Q6_K> {
       hi[k] = ds1 * (float)(qh - 32);
     }
     return pk_word_kinds(lo, xv) | pk_word_kinds(hi, xw);
+  }
+};
+
+// The same decodes on the GGUF payload itself (T | PK_GGUF): one region, the
+// rows as stored, a lane's code bytes found inside the blocks instead of in
+// the code stream.  Blocks of 18, 22, 34 and 210 bytes put the 16-byte loads
+// on any even address, which the parts take in the unaligned access mode the
+// HSA runtime sets; 64 lanes still cover one contiguous span of blocks.
+// Against the kernels this replaces (wavefront- or tile-staged: each byte
+// through LDS both ways), eager calls: Q8_0 4096 x 4096 6.6 -> 5.5 us, 4096 x
+// 14336 16.3 -> 12.3; Q4_0 14336 x 4096 11.0 -> 8.9; Q5_0 19.6 -> 10.4; Q4_K
+// 14.0 -> 9.1, 4096 x 14336 18.8 -> 10.8; Q5_K 14336 x 4096 21.5 -> 11.0;
+// Q6_K 16.2 -> 11.9, 128256 x 4096 114 -> 92.  Non-temporal loads, which suit
+// the packed regions, are slower here (Q8_0 14336 x 4096 14.1): neighbouring
+// loads share cache lines.
+constexpr uint32_t PK_GGUF = 0x100;
+__host__ __device__ constexpr uint32_t pk_base(uint32_t t) { return t & 0xFFu; }
+
+template <> struct PkFmt<T_Q8_0 | PK_GGUF> : PkFmt<T_Q8_0> {
+  static constexpr uint32_t NREG = 1;
+  static constexpr bool INTX = false;
+  __host__ __device__ static uint64_t row_bytes(int, uint64_t in) { return in / 32 * 34; }
+  __device__ static void fetch(nv_u32x4& q, Meta& m, const PkRsrc* r, uint32_t b) {
+    const uint32_t o = (b >> 5) * 34u;
+    q = __builtin_amdgcn_raw_buffer_load_b128(r[0], o + 2u + (b & 31u), 0, 0);
+    m = __builtin_amdgcn_raw_buffer_load_b16(r[0], o, 0, 0);
+  }
+};
+template <> struct PkFmt<T_Q4_0 | PK_GGUF> : PkFmt<T_Q4_0> {
+  static constexpr uint32_t NREG = 1;
+  static constexpr bool INTX = false;
+  __host__ __device__ static uint64_t row_bytes(int, uint64_t in) { return in / 32 * 18; }
+  __device__ static void fetch(nv_u32x4& q, Meta& m, const PkRsrc* r, uint32_t b) {
+    const uint32_t o = (b >> 4) * 18u;
+    q = __builtin_amdgcn_raw_buffer_load_b128(r[0], o + 2u, 0, 0);
+    m = __builtin_amdgcn_raw_buffer_load_b16(r[0], o, 0, 0);
+  }
+};
+template <> struct PkFmt<T_Q4_K | PK_GGUF> : PkFmt<T_Q4_K> {
+  static constexpr uint32_t NREG = 1;
+  __host__ __device__ static uint64_t row_bytes(int, uint64_t in) { return in / 256 * 144; }
+  __device__ static void fetch(nv_u32x4& q, Meta& m, const PkRsrc* r, uint32_t b) {
+    const uint32_t o = (b >> 7) * 144u;
+    q = __builtin_amdgcn_raw_buffer_load_b128(r[0], o + 16u + (b & 127u), 0, 0);
+    m = __builtin_amdgcn_raw_buffer_load_b128(r[0], o, 0, 0);
+  }
+};
+template <> struct PkFmt<T_Q6_K | PK_GGUF> : PkFmt<T_Q6_K> {
+  static constexpr uint32_t NREG = 1;
+  __host__ __device__ static uint64_t row_bytes(int, uint64_t in) { return in / 256 * 210; }
+  __device__ static void fetch(nv_u32x4& q, Meta& m, const PkRsrc* r, uint32_t b) {
+    const uint32_t base = (b >> 7) * 210u, o = b & 127u;
+    q = __builtin_amdgcn_raw_buffer_load_b128(r[0], base + o, 0, 0);
+    m.qh = __builtin_amdgcn_raw_buffer_load_b128(r[0], base + 128u + 32u * (o >> 6) + (o & 31u), 0, 0);
+    m.sc = __builtin_amdgcn_raw_buffer_load_b128(r[0], base + 192u, 0, 0);
+    m.d = __builtin_amdgcn_raw_buffer_load_b16(r[0], base + 208u, 0, 0);
+  }
+};
+// Q5_0 (quant.rs:117-151): d, qh (bit e of element e), 16 bytes of nibbles; a
+// lane's 16 bytes are one block, as in Q4_0.
+template <> struct PkFmt<T_Q5_0 | PK_GGUF> : PkFmt<T_Q4_0 | PK_GGUF> {
+  struct Meta {
+    uint32_t d, qh;
+  };
+  __host__ __device__ static uint64_t row_bytes(int, uint64_t in) { return in / 32 * 22; }
+  __device__ static void fetch(nv_u32x4& q, Meta& m, const PkRsrc* r, uint32_t b) {
+    const uint32_t o = (b >> 4) * 22u;
+    q = __builtin_amdgcn_raw_buffer_load_b128(r[0], o + 6u, 0, 0);
+    m.qh = __builtin_amdgcn_raw_buffer_load_b32(r[0], o + 2u, 0, 0);
+    m.d = __builtin_amdgcn_raw_buffer_load_b16(r[0], o, 0, 0);
+  }
+  // bits 4 i .. 4 i + 3 of h as bit 4 of four bytes
+  __device__ static uint32_t spread(uint32_t h, int i) {
+    return ((((h >> (4 * i)) & 0xFu) * 0x00204081u) & 0x01010101u) << 4;
+  }
+  // the codes q - 16 as int8 bytes 8 (q - 16), the factor 8 off in finish
+  __device__ static void word(const Lane&, uint32_t q, const Meta& m, int i, const float4& xv, const float4& xw,
+                              float& s0, float& s1) {
+    const uint32_t lo = rf_opaque(rf_top_signed((q & 0x0F0F0F0Fu) | spread(m.qh, i), 5));
+    const uint32_t hi = rf_opaque(rf_top_signed(((q >> 4) & 0x0F0F0F0Fu) | spread(m.qh >> 16, i), 5));
+    s0 = fmaf(rf_sb(lo, 0), xv.x, s0); s0 = fmaf(rf_sb(lo, 1), xv.y, s0);
+    s0 = fmaf(rf_sb(lo, 2), xv.z, s0); s0 = fmaf(rf_sb(lo, 3), xv.w, s0);
+    s1 = fmaf(rf_sb(hi, 0), xw.x, s1); s1 = fmaf(rf_sb(hi, 1), xw.y, s1);
+    s1 = fmaf(rf_sb(hi, 2), xw.z, s1); s1 = fmaf(rf_sb(hi, 3), xw.w, s1);
+  }
+  __device__ static float finish(const Lane&, const nv_u32x4&, const Meta& m, float s0, float s1, float, float) {
+    return rf_half_to_float_fast(m.d) * ((s0 + s1) * 0.125f);
+  }
+};
+// Q5_K (quant.rs:259-343): Q4_K's header, qh[32], qs[128].  Element l of
+// sub-block s has its high bit in bit s of qh[8 (s / 2) + l / 8] (the
+// reference's own index), so the two bytes 8 g + 2 hh, + 1 serve a lane's
+// half hh of group g: byte i / 2 for word i, bit 2 g for the low nibbles'
+// sub-block and 2 g + 1 for the high ones'.
+template <> struct PkFmt<T_Q5_K | PK_GGUF> : PkFmt<T_Q4_K | PK_GGUF> {
+  struct Meta {
+    nv_u32x4 h;
+    uint32_t qh;
+  };
+  struct Lane : PkFmt<T_Q4_K>::Lane {
+    uint32_t bit;  // 2 g
+    __device__ explicit Lane(uint32_t lane) : PkFmt<T_Q4_K>::Lane(lane), bit(lane & 6u) {}
+  };
+  __host__ __device__ static uint64_t row_bytes(int, uint64_t in) { return in / 256 * 176; }
+  __device__ static void fetch(nv_u32x4& q, Meta& m, const PkRsrc* r, uint32_t b) {
+    const uint32_t base = (b >> 7) * 176u, o = b & 127u;
+    q = __builtin_amdgcn_raw_buffer_load_b128(r[0], base + 48u + o, 0, 0);
+    m.h = __builtin_amdgcn_raw_buffer_load_b128(r[0], base, 0, 0);
+    m.qh = __builtin_amdgcn_raw_buffer_load_b16(r[0], base + 16u + 8u * (o >> 5) + 2u * ((o >> 4) & 1u), 0, 0);
+  }
+  __device__ static uint32_t high(const Lane& L, const Meta& m, int i, int h) {
+    return ((m.qh >> (8 * (i >> 1))) >> (L.bit + h)) & 1u;
+  }
+  __device__ static void word(const Lane& L, uint32_t q, const Meta& m, int i, const float4& xv, const float4& xw,
+                              float& s0, float& s1) {
+    const uint32_t lo = rf_opaque((q & 0x0F0F0F0Fu) | (high(L, m, i, 0) * 0x10101010u));
+    const uint32_t hi = rf_opaque(((q >> 4) & 0x0F0F0F0Fu) | (high(L, m, i, 1) * 0x10101010u));
+    s0 = fmaf(rf_ub(lo, 0), xv.x, s0); s0 = fmaf(rf_ub(lo, 1), xv.y, s0);
+    s0 = fmaf(rf_ub(lo, 2), xv.z, s0); s0 = fmaf(rf_ub(lo, 3), xv.w, s0);
+    s1 = fmaf(rf_ub(hi, 0), xw.x, s1); s1 = fmaf(rf_ub(hi, 1), xw.y, s1);
+    s1 = fmaf(rf_ub(hi, 2), xw.z, s1); s1 = fmaf(rf_ub(hi, 3), xw.w, s1);
+  }
+  __device__ static float finish(const Lane& L, const nv_u32x4& q, const Meta& m, float s0, float s1, float xs0, float xs1) {
+    return PkFmt<T_Q4_K>::finish(L, q, m.h, s0, s1, xs0, xs1);
+  }
+  __device__ static uint32_t kinds(const Lane& L, uint32_t q, const Meta& m, int i, const float4& xv, const float4& xw) {
+    uint32_t out = 0;
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+      float d1, m1, deq[4];
+      PkFmt<T_Q4_K>::scale_min(L, m.h, h, d1, m1);
+#pragma unroll
+      for (int k = 0; k < 4; ++k) {
+        const float prod = d1 * (float)(((q >> (8 * k + 4 * h)) & 0xFu) | (high(L, m, i, h) << 4));
+        deq[k] = __fsub_rn(prod, m1);
+      }
+      out |= pk_word_kinds(deq, h ? xw : xv);
+    }
+    return out;
+  }
+};
+
+// Rows of an even number of such blocks on a dword-aligned base (T | PK_GGUF |
+// PK_DWORD): a pair of blocks is whole dwords, its first block's codes start
+// two bytes into one.  The loads take whole dwords and the decode realigns
+// them (code(), one v_alignbyte per word): a half-aligned 16-byte load costs
+// about twice an aligned one (Q8_0 128256 x 4096 134 against 99 us).
+constexpr uint32_t PK_DWORD = 0x200;
+__device__ __forceinline__ uint32_t pk_realign(uint32_t lo, uint32_t hi, uint32_t sh) {
+  return __builtin_amdgcn_alignbyte(hi, lo, sh);
+}
+// Q8_0, 17 dwords a pair: four lanes take dwords 0-3, 4-7 (first block: scale,
+// then codes), 9-12, 13-16 (second block's codes); dword 8, the first block's
+// last codes and the second's scale, goes to all four, and the first block's
+// scale and the dword its first lane lacks come from the neighbour.
+template <> struct PkFmt<T_Q8_0 | PK_GGUF | PK_DWORD> : PkFmt<T_Q8_0 | PK_GGUF> {
+  struct Lane {
+    uint32_t sh;
+    bool first;
+    __device__ explicit Lane(uint32_t lane) : sh((lane & 2u) ? 0u : 2u), first((lane & 3u) == 0u) {}
+  };
+  __device__ static void fetch(nv_u32x4& q, Meta& m, const PkRsrc* r, uint32_t b) {
+    const uint32_t o = (b >> 6) * 68u, j = (b >> 4) & 3u;
+    q = __builtin_amdgcn_raw_buffer_load_b128(r[0], o + 16u * j + 4u * (j >> 1), 0, 0);
+    m = __builtin_amdgcn_raw_buffer_load_b32(r[0], o + 32u, 0, 0);
+  }
+  // q[0] of lane 1 (0) of the quad to lane 0 (1)
+  __device__ static uint32_t swap(uint32_t v) { return (uint32_t)__builtin_amdgcn_mov_dpp((int)v, 0xE1, 0xF, 0xF, true); }
+  __device__ static uint32_t code(const Lane& L, const nv_u32x4& q, const Meta& m, int i) {
+    if (i < 3) return pk_realign(q[i], q[i + 1], L.sh);  // i is a compile-time index
+    const uint32_t n = swap(q[0]);  // by all lanes
+    return pk_realign(q[i], L.first ? n : m, L.sh);
+  }
+  __device__ static void word(const Lane&, uint32_t q, const Meta&, int, const float4& xv, const float4& xw, float& s0,
+                              float& s1) {
+    PkFmt<T_Q8_0>::word(PkFmt<T_Q8_0>::Lane(0), q, 0u, 0, xv, xw, s0, s1);
+  }
+  __device__ static float finish(const Lane& L, const nv_u32x4& q, const Meta& m, float s0, float, float, float) {
+    const uint32_t n = swap(q[0]);
+    const uint32_t d = L.sh == 0u ? m >> 16 : (L.first ? q[0] : n) & 0xFFFFu;
+    return rf_half_to_float_fast(d) * s0;
+  }
+};
+// Q4_0, 9 dwords a pair: a lane each, dwords 0-3 and 5-8, dword 4 to both.
+template <> struct PkFmt<T_Q4_0 | PK_GGUF | PK_DWORD> : PkFmt<T_Q4_0 | PK_GGUF> {
+  struct Lane {
+    uint32_t sh;
+    __device__ explicit Lane(uint32_t lane) : sh((lane & 1u) ? 0u : 2u) {}
+  };
+  __device__ static void fetch(nv_u32x4& q, Meta& m, const PkRsrc* r, uint32_t b) {
+    const uint32_t o = (b >> 5) * 36u;
+    q = __builtin_amdgcn_raw_buffer_load_b128(r[0], o + 20u * ((b >> 4) & 1u), 0, 0);
+    m = __builtin_amdgcn_raw_buffer_load_b32(r[0], o + 16u, 0, 0);
+  }
+  __device__ static uint32_t code(const Lane& L, const nv_u32x4& q, const Meta& m, int i) {
+    return pk_realign(q[i], i < 3 ? q[i + 1] : m, L.sh);
+  }
+  __device__ static void word(const Lane&, uint32_t q, const Meta&, int, const float4& xv, const float4& xw, float& s0,
+                              float& s1) {
+    PkFmt<T_Q4_0>::word(PkFmt<T_Q4_0>::Lane(0), q, 0u, 0, xv, xw, s0, s1);
+  }
+  __device__ static float finish(const Lane& L, const nv_u32x4& q, const Meta& m, float s0, float s1, float, float) {
+    const uint32_t d = L.sh == 0u ? m >> 16 : q[0] & 0xFFFFu;
+    return rf_half_to_float_fast(d) * ((s0 + s1) * 0.0625f);
+  }
+};
+// Q6_K: a block starts 0 or 2 bytes into a dword by its parity, a lane constant.
+template <> struct PkFmt<T_Q6_K | PK_GGUF | PK_DWORD> : PkFmt<T_Q6_K | PK_GGUF> {
+  struct Meta {
+    nv_u32x4 qh;
+    uint32_t tail, htail, sc[3], d;
+  };
+  struct Lane : PkFmt<T_Q6_K>::Lane {
+    uint32_t sh;
+    __device__ explicit Lane(uint32_t lane) : PkFmt<T_Q6_K>::Lane(lane), sh((lane & 8u) ? 2u : 0u) {}
+  };
+  __device__ static void fetch(nv_u32x4& q, Meta& m, const PkRsrc* r, uint32_t b) {
+    const uint32_t base = (b >> 7) * 210u, o = b & 127u, ab = base & ~3u, h = ab + 128u + 32u * (o >> 6) + (o & 31u);
+    q = __builtin_amdgcn_raw_buffer_load_b128(r[0], ab + o, 0, 0);
+    m.tail = __builtin_amdgcn_raw_buffer_load_b32(r[0], ab + o + 16u, 0, 0);
+    m.qh = __builtin_amdgcn_raw_buffer_load_b128(r[0], h, 0, 0);
+    m.htail = __builtin_amdgcn_raw_buffer_load_b32(r[0], h + 16u, 0, 0);
+    const auto sc = __builtin_amdgcn_raw_buffer_load_b96(r[0], ab + 192u + 8u * (o >> 6), 0, 0);
+    m.sc[0] = sc[0]; m.sc[1] = sc[1]; m.sc[2] = sc[2];
+    m.d = __builtin_amdgcn_raw_buffer_load_b16(r[0], base + 208u, 0, 0);
+  }
+  __device__ static uint32_t code(const Lane& L, const nv_u32x4& q, const Meta& m, int i) {
+    return pk_realign(q[i], i < 3 ? q[i + 1] : m.tail, L.sh);
+  }
+  __device__ static void word(const Lane& L, uint32_t q, const Meta& m, int i, const float4& xv, const float4& xw,
+                              float& s0, float& s1) {
+    PkFmt<T_Q6_K>::Meta w;
+    w.qh[i] = pk_realign(m.qh[i], i < 3 ? m.qh[i + 1] : m.htail, L.sh);
+    PkFmt<T_Q6_K>::word(L, q, w, i, xv, xw, s0, s1);
+  }
+  __device__ static float finish(const Lane& L, const nv_u32x4&, const Meta& m, float s0, float s1, float, float) {
+    const uint32_t w0 = pk_realign(m.sc[0], m.sc[1], L.sh), w1 = pk_realign(m.sc[1], m.sc[2], L.sh);
+    return rf_half_to_float_fast(m.d) * (fmaf(rf_sb(w0 >> L.bsh, 0), s0, rf_sb(w1 >> L.bsh, 0) * s1) * 0.25f);
   }
 };
 
@@ -378,604 +626,38 @@ struct PkStep {
 template <uint32_t T, int EPI, bool NORM, int U, int LPW, int NB, int NT, bool IX, bool ALLF = false,
           bool MRG = false>
 __global__ __launch_bounds__(NT) void matvec_packed(PkArgs a) {
-  typedef PkFmt<T> F;
-  constexpr bool IXE = F::INTX && IX;  // digit planes instead of float x
-  static_assert(!MRG || (!IXE && !NORM && EPI == EPI_RESIDUAL && ALLF), "merged x: one float-x residual step");
-  // Non-finite x needs a fallback only where a decode does not multiply each
-  // signed code by x: the digit planes, and Q4_K's min term (d sc sum(q x) -
-  // dmin m sum(x) gives inf - inf where the reference's (d sc q - dmin m) x
-  // is an infinity).  The signed-code float decodes of Q8_0, Q4_0 and Q6_K
-  // produce the reference's NaN / +-inf rows by themselves: a code times an
-  // infinity is the reference's term up to a positive power of two, and
-  // finite terms cannot change an infinite or NaN sum.
-  constexpr bool KINDS = IXE || T == T_Q4_K;
-  constexpr bool DUAL = EPI == EPI_SWIGLU;
-  constexpr uint32_t EPB = F::EPB, UPS = EPB, EPL = 16u * UPS, NW = NT / 64;
-  extern __shared__ __align__(16) float xl[];  // [nchunk * 64 * EPL] x, then [nchunk * 64 * UPS] unit sums
-  __shared__ float wsum[NW];
-  __shared__ uint32_t wbad[NW];  // the wavefront staged a non-finite x element
-  __shared__ float resl[EPI == EPI_RESIDUAL ? NW : 1][PK_RES_SLOTS][U];
-  static_assert(sizeof(wsum) + sizeof(wbad) + sizeof(resl) <= PK_STATIC_LDS,
-                "static LDS above the planner's reservation");
-  // The wavefront index through readfirstlane: rows, segments and their
-  // pointers are then scalar values, so no vector load (whose wait would also
-  // wait for the codes in flight) is spent on them.
-  const uint32_t tid = threadIdx.x, lane = tid & 63u, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-  // MRG: the position first, before any store of the kernel (so that it is a
-  // scalar load: nothing this kernel writes comes before it)
-  const uint32_t m_posv = MRG ? (uint32_t)(*a.m_pos) : 0u;
-  if (a.advance != nullptr && blockIdx.x == 0 && tid == 0) *a.advance += 1;
-  const uint32_t in = a.in_dim, crb = in / EPB;
-  const uint32_t nchunk = (crb + 1023u) / 1024u, nstep = (nchunk + LPW - 1) / LPW;
-  float* xsum_l = xl + nchunk * 64u * EPL;
-  // INTX: digit planes (plane p of unit h of lane l in chunk c at byte
-  // ((c UPS + h) PK_PLANES + p) 1024 + 16 l), then (scale, scale * sum of X)
-  // of unit j at float2 j.  The launch sizes LDS for the larger of this and
-  // the float layout, which the kernel falls back to for a non-finite x.
-  uint8_t* xdig = reinterpret_cast<uint8_t*>(xl);
-  float2* xinfo = reinterpret_cast<float2*>(xdig + nchunk * UPS * (1024u * PK_PLANES));
-  const typename F::Lane LC(lane);
-
   auto seg_of = [&](uint32_t v) -> PkSeg {
     return (a.nseg > 2 && v >= a.seg[2].row_begin) ? a.seg[2]
                                                    : ((a.nseg > 1 && v >= a.seg[1].row_begin) ? a.seg[1] : a.seg[0]);
   };
+#include "rf_matvec_packed_body.inc"
+}
 
-  const uint32_t ntask = (a.rows_total + U - 1) / U;
-  const uint32_t gstride = gridDim.x * NW;
-
-  typedef PkStep<T, U, LPW, DUAL> Step;
-  Step buf[NB];
-  // Raw buffer loads: one resource per row and region (scalar base, range =
-  // the row's bytes), the lane's byte offset in a VGPR.  Offsets past the row
-  // (the tail of a partial chunk) and every load of a fetch past the last task
-  // (range 0) return zeros without touching memory, so fetches are issued
-  // unconditionally and the compiler's wait counts stay exact: a consume waits
-  // for its own step only, never for the prefetch behind it.
-  auto fetch = [&](Step& B, uint32_t t, uint32_t st) {
-    const bool live = t < ntask;  // wave-uniform
-#pragma unroll
-    for (int u = 0; u < U; ++u) {
-      const uint32_t v = min(t * U + u, a.rows_total - 1u);
-      const PkSeg g = seg_of(v);
-      const uint32_t r = v - g.row_begin;
-      PkRsrc rr[F::NREG], rr2[F::NREG];
-#pragma unroll
-      for (int k = 0; k < (int)F::NREG; ++k) {
-        const uint32_t rb = (uint32_t)F::row_bytes(k, in);
-        const int32_t n = live ? (int32_t)rb : 0;
-        rr[k] = __builtin_amdgcn_make_buffer_rsrc((void*)(g.reg[k] + (size_t)r * rb), 0, n, PK_RSRC_WORD3);
-        if constexpr (DUAL)
-          rr2[k] = __builtin_amdgcn_make_buffer_rsrc((void*)(g.reg_up[k] + (size_t)r * rb), 0, n, PK_RSRC_WORD3);
-      }
-#pragma unroll
-      for (int l = 0; l < LPW; ++l) {
-        const uint32_t b = (st * LPW + l) * 1024u + 16u * lane;
-        F::fetch(B.q[u][l], B.m[u][l], rr, b);
-        if constexpr (DUAL) F::fetch(B.q2[u][l], B.m2[u][l], rr2, b);
-      }
-    }
+// A plain y = W x on GGUF bytes with just its own arguments: the 350 bytes of
+// PkArgs cost an eager call 0.3 us on the host.  (One body behind a device
+// function that takes the arguments by reference puts them in scratch memory:
+// 8B decode 34 -> 43 ms.)
+struct PkPlainArgs {
+  const uint8_t* w;
+  const float* x;
+  float* y;
+  uint32_t rows_total, in_dim;
+  static constexpr const float *norm_w = nullptr, *mws = nullptr;
+  static constexpr int32_t *advance = nullptr, *m_pos = nullptr;
+  static constexpr float eps = 0.f;
+  static constexpr uint32_t m_nsplit = 0, m_qh = 0, m_hd_log2 = 0;
+};
+template <uint32_t T, int LPW, int NB, int NT, bool ALLF>
+__global__ __launch_bounds__(NT) void matvec_gguf(PkPlainArgs a) {
+  constexpr int EPI = EPI_STORE, U = 1;
+  constexpr bool NORM = false, IX = false, MRG = false;
+  auto seg_of = [&](uint32_t) {
+    PkSeg g{};
+    g.reg[0] = a.w;
+    g.y = a.y;
+    return g;
   };
-
-  auto advance = [&](uint32_t& tt, uint32_t& ss) {
-    if (++ss == nstep) { ss = 0; tt += gstride; }
-  };
-  // Prologue, one round of loads and one barrier.  Thread j (then j + NT, ...)
-  // owns unit j: 16 consecutive elements of x, unit j % UPS of lane slice
-  // j / UPS.  It writes the unit into LDS and the unit's sum.  With NORM,
-  // rms_norm_reference (core/src/compute.rs:291-319) is
-  // x / sqrt(mean(x^2) + eps) * w; LDS holds x * w and every row sum is
-  // scaled by 1 / sqrt(mean(x^2) + eps) in the epilogue (the same value up to
-  // rounding), so the mean's reduction shares the prologue's barrier.
-  const uint32_t nunit = nchunk * 64u * UPS;
-  const float4* x4 = reinterpret_cast<const float4*>(a.x);
-  const float4* w4 = reinterpret_cast<const float4*>(a.norm_w);
-  // The 16 elements of unit j (times the norm weights), their squares summed
-  // into ss; false for the zero padding past the row.
-  auto load_unit = [&](uint32_t j, float* v, float& ss, bool sq) -> bool {
-    const uint32_t js = j / UPS, h = j % UPS;
-    const uint32_t b = (js >> 6) * 1024u + 16u * (js & 63u);
-    if (b >= crb) return false;
-    const uint32_t e = F::unit_elem(b, h);
-#pragma unroll
-    for (int k = 0; k < 4; ++k) {
-      const float4 xv = x4[e / 4u + k];
-      v[4 * k] = xv.x; v[4 * k + 1] = xv.y; v[4 * k + 2] = xv.z; v[4 * k + 3] = xv.w;
-      if (NORM) {
-        const float4 wv = w4[e / 4u + k];
-        if (sq) {
-          ss = fmaf(xv.x, xv.x, ss); ss = fmaf(xv.y, xv.y, ss);
-          ss = fmaf(xv.z, xv.z, ss); ss = fmaf(xv.w, xv.w, ss);
-        }
-        v[4 * k] *= wv.x; v[4 * k + 1] *= wv.y; v[4 * k + 2] *= wv.z; v[4 * k + 3] *= wv.w;
-      }
-    }
-    return true;
-  };
-  // Float layout: unit j (values v, or the zero padding past the row when
-  // !have) in its permuted LDS slots and its sum.  Returns false for a
-  // non-finite element.
-  auto put_float = [&](uint32_t j, const float* v, bool have, bool check) -> bool {
-    const uint32_t js = j / UPS, h = j % UPS;
-    float s = 0.f;
-    bool fin = true;
-    if (have) {
-      float* dst = xl + (js >> 6) * 64u * EPL + 4u * h * 256u + 4u * (js & 63u);
-#pragma unroll
-      for (int k = 0; k < 4; ++k) {
-        *reinterpret_cast<float4*>(dst + 256 * k) = make_float4(v[4 * k], v[4 * k + 1], v[4 * k + 2], v[4 * k + 3]);
-        s += v[4 * k]; s += v[4 * k + 1]; s += v[4 * k + 2]; s += v[4 * k + 3];
-      }
-      if (check) {
-#pragma unroll
-        for (int k = 0; k < 16; ++k) fin = fin && fabsf(v[k]) <= 3.40282347e38f;
-      }
-    }
-    xsum_l[j] = s;
-    return fin;
-  };
-  auto stage_float = [&](uint32_t j, float& ss, bool sq, bool check) -> bool {
-    float v[16];
-    const bool have = load_unit(j, v, ss, sq);
-    return put_float(j, v, have, check);
-  };
-  // Digit layout: with 2^E above the unit's largest |x|, X = rint(x 2^(30 - E))
-  // (|X| < 2^30) in balanced base-256 digits X = 2^24 a + 2^16 b + 2^8 c + e
-  // (a in [-64, 64]); codes times digits then sum exactly in int32.  Each
-  // element is off by at most 2^(E - 31), i.e. x keeps 30 bits below the
-  // unit's largest element.  E is at least -96 so the scale 2^(E - 30) is a
-  // normal float.  Returns false for a non-finite element (the kernel then
-  // restages x as floats).
-  auto stage_digits = [&](uint32_t j, float& ss) -> bool {
-    const uint32_t js = j / UPS, h = j % UPS;
-    nv_u32x4 pl[PK_PLANES] = {};
-    float2 info = make_float2(0.f, 0.f);
-    float v[16];
-    bool fin = true;
-    if (load_unit(j, v, ss, true)) {
-      float mx = 0.f;
-#pragma unroll
-      for (int k = 0; k < 16; ++k) {
-        mx = fmaxf(mx, fabsf(v[k]));
-        fin = fin && fabsf(v[k]) <= 3.40282347e38f;
-      }
-      int ex = 0;
-      (void)frexpf(mx, &ex);
-      ex = ex < -96 ? -96 : ex;
-      long long sx = 0;
-#pragma unroll
-      for (int k = 0; k < 16; ++k) {
-        const int X = fin ? (int)rintf(ldexpf(v[k], 30 - ex)) : 0;
-        const int d0 = (int)(int8_t)(X & 0xFF), X1 = (X - d0) >> 8;
-        const int c0 = (int)(int8_t)(X1 & 0xFF), X2 = (X1 - c0) >> 8;
-        const int b0 = (int)(int8_t)(X2 & 0xFF), a0 = (X2 - b0) >> 8;
-        sx += X;
-        const int sh = 8 * (k & 3);
-        pl[0][k >> 2] |= (uint32_t)(a0 & 0xFF) << sh;
-        pl[1][k >> 2] |= (uint32_t)(b0 & 0xFF) << sh;
-        pl[2][k >> 2] |= (uint32_t)(c0 & 0xFF) << sh;
-        pl[3][k >> 2] |= (uint32_t)(d0 & 0xFF) << sh;
-      }
-      const float sc = ldexpf(1.f, ex - 30);
-      info = make_float2(sc, sc * (float)sx);
-    }
-    uint8_t* dst = xdig + (((js >> 6) * UPS + h) * PK_PLANES) * 1024u + 16u * (js & 63u);
-#pragma unroll
-    for (int p = 0; p < PK_PLANES; ++p) *reinterpret_cast<nv_u32x4*>(dst + 1024u * p) = pl[p];
-    xinfo[j] = info;
-    return fin;
-  };
-
-  // MRG: the (m, l) pair of record tid, then this thread's half of its unit
-  // (thread t: unit t / 2, elements 8 (t % 2) .. + 7) from every chunk, all
-  // before the weights.  Only the valid chunks' records are read (a uniform
-  // count); with a single chunk the attention wrote x itself.
-  uint32_t m_ns = 1, m_head = 0;
-  float2 mlv = make_float2(0.f, 0.f);
-  float4 mo[MRG ? 8 : 1][2];
-  if constexpr (MRG) {
-    const uint32_t total = m_posv + 1u, chunk = att_chunk(total, a.m_nsplit);
-    m_ns = (total + chunk - 1u) / chunk;
-    const uint32_t rec = att_rec(1u << a.m_hd_log2), hmask = (1u << a.m_hd_log2) - 1u;
-    const PkRsrc wsr =
-        __builtin_amdgcn_make_buffer_rsrc((void*)a.mws, 0, (int32_t)(m_ns * a.m_qh * rec * 4u), PK_RSRC_WORD3);
-    // lanes 8 h .. 8 h + 7: head h's (m, l) of chunks 0..7 (m = -inf, l = 0
-    // past the valid ones)
-    mlv = make_float2(-INFINITY, 0.f);
-    if (m_ns > 1u && (tid >> 3) < a.m_qh && (tid & 7u) < m_ns) {
-      const uint32_t r = (tid & 7u) * a.m_qh + (tid >> 3);
-      const auto v = __builtin_amdgcn_raw_buffer_load_b64(wsr, (r * rec + hmask + 1u) * 4u, 0, 0);
-      mlv = make_float2(__uint_as_float(v[0]), __uint_as_float(v[1]));
-    }
-    const uint32_t j = tid >> 1, js = j / UPS, hh = j % UPS;
-    const uint32_t b = (js >> 6) * 1024u + 16u * (js & 63u);
-    const uint32_t e = (j < nunit && b < crb ? F::unit_elem(b, hh) : 0u) + 8u * (tid & 1u);
-    m_head = e >> a.m_hd_log2;
-    if (m_ns == 1u) {
-      const float4* xs = reinterpret_cast<const float4*>(a.x) + e / 4u;
-      mo[0][0] = xs[0];
-      mo[0][1] = xs[1];
-    } else {
-      const uint32_t off = ((m_head * rec) + (e & hmask)) * 4u, cstride = a.m_qh * rec * 4u;
-#pragma unroll
-      for (int c = 0; c < 8; ++c) {
-        if ((uint32_t)c < m_ns) {  // uniform
-#pragma unroll
-          for (int k = 0; k < 2; ++k) {
-            const auto v = __builtin_amdgcn_raw_buffer_load_b128(wsr, off + c * cstride + 16u * k, 0, 0);
-            mo[c][k] = make_float4(__uint_as_float(v[0]), __uint_as_float(v[1]), __uint_as_float(v[2]),
-                                   __uint_as_float(v[3]));
-          }
-        }
-      }
-    }
-  }
-  // x first: the raw loads of this thread's first unit are issued before
-  // any weight step, so the prologue's wait for them does not also wait for
-  // the codes requested behind them (a wavefront's loads complete in order).
-  float4 xr[4], wr[4];
-  bool xin = false;
-  if constexpr (!IXE && !MRG) {
-    const uint32_t js = tid / UPS, h = tid % UPS;
-    const uint32_t b = (js >> 6) * 1024u + 16u * (js & 63u);
-    xin = tid < nunit && b < crb;
-    if (xin) {
-      const uint32_t e = F::unit_elem(b, h);
-#pragma unroll
-      for (int k = 0; k < 4; ++k) {
-        xr[k] = x4[e / 4u + k];
-        if (NORM) wr[k] = w4[e / 4u + k];
-      }
-    }
-  }
-  // (Loading the first task's residual here too, before the weights, made
-  // the 8B down projection 2.5 us slower.)
-  __builtin_amdgcn_sched_barrier(0);
-  // The first NB - 1 steps (ALLF: all NB) are requested before the prologue.
-  uint32_t ct = blockIdx.x * NW + wave, cs = 0, ft = ct, fs = 0;
-#pragma unroll
-  for (int b = 0; b < (ALLF ? NB : NB - 1); ++b) {
-    fetch(buf[b], ft, fs);
-    advance(ft, fs);
-  }
-
-  bool finite = true;
-  if constexpr (MRG) {
-    // The merge's per-record work once per workgroup: each group of 8 lanes
-    // holds one head's chunks, so M = the largest m, the factors exp(m - M)
-    // and L = the sum of l times factor (a fixed butterfly order) take three
-    // lane exchanges each; the factors and 1 / L go to LDS behind the unit
-    // sums.  Each thread then sums factor times o over the chunks for its 8
-    // elements, scales by 1 / L and stages them.
-    float* fac = xsum_l + nunit;                 // [nsplit][qh]
-    float* invl = fac + a.m_nsplit * a.m_qh;     // [qh]
-    if (m_ns > 1u) {
-      float M = mlv.x;
-      M = fmaxf(M, __shfl_xor(M, 1));
-      M = fmaxf(M, __shfl_xor(M, 2));
-      M = fmaxf(M, __shfl_xor(M, 4));
-      const float f = expf(mlv.x - M);  // 0 past the valid chunks
-      float L = mlv.y * f;
-      L += __shfl_xor(L, 1);
-      L += __shfl_xor(L, 2);
-      L += __shfl_xor(L, 4);
-      const uint32_t h = tid >> 3, c = tid & 7u;
-      if (h < a.m_qh) {
-        if (c < m_ns) fac[c * a.m_qh + h] = f;
-        if (c == 0u) invl[h] = 1.0f / L;
-      }
-      __syncthreads();
-    }
-    const uint32_t j = tid >> 1, half = tid & 1u, js = j / UPS, hh = j % UPS;
-    const bool have = j < nunit && (js >> 6) * 1024u + 16u * (js & 63u) < crb;
-    float v[8];
-    if (m_ns == 1u) {
-#pragma unroll
-      for (int k = 0; k < 2; ++k) {
-        v[4 * k] = mo[0][k].x; v[4 * k + 1] = mo[0][k].y; v[4 * k + 2] = mo[0][k].z; v[4 * k + 3] = mo[0][k].w;
-      }
-    } else {
-      const float f0 = fac[m_head];  // chunk 0 (m_ns >= 2)
-#pragma unroll
-      for (int k = 0; k < 2; ++k) {
-        v[4 * k] = f0 * mo[0][k].x; v[4 * k + 1] = f0 * mo[0][k].y;
-        v[4 * k + 2] = f0 * mo[0][k].z; v[4 * k + 3] = f0 * mo[0][k].w;
-      }
-#pragma unroll
-      for (int c = 1; c < 8; ++c) {
-        if ((uint32_t)c < m_ns) {
-          const float f = fac[c * a.m_qh + m_head];
-#pragma unroll
-          for (int k = 0; k < 2; ++k) {
-            v[4 * k] = fmaf(f, mo[c][k].x, v[4 * k]);
-            v[4 * k + 1] = fmaf(f, mo[c][k].y, v[4 * k + 1]);
-            v[4 * k + 2] = fmaf(f, mo[c][k].z, v[4 * k + 2]);
-            v[4 * k + 3] = fmaf(f, mo[c][k].w, v[4 * k + 3]);
-          }
-        }
-      }
-      const float r = invl[m_head];
-#pragma unroll
-      for (int k = 0; k < 8; ++k) v[k] *= r;
-    }
-    // the unit's slots (put_float's layout): this half's two float4; the
-    // unit's sum (the two halves, adjacent lanes) where the format reads it
-    if (have) {
-      float* dst = xl + (js >> 6) * 64u * EPL + 4u * hh * 256u + 4u * (js & 63u) + 512u * half;
-#pragma unroll
-      for (int k = 0; k < 2; ++k)
-        *reinterpret_cast<float4*>(dst + 256 * k) = make_float4(v[4 * k], v[4 * k + 1], v[4 * k + 2], v[4 * k + 3]);
-    }
-    if constexpr (T == T_Q4_K) {
-      float s8 = 0.f;
-#pragma unroll
-      for (int k = 0; k < 8; ++k) s8 += v[k];
-      const float s16 = s8 + __shfl_xor(s8, 1);
-      if (j < nunit && half == 0u) xsum_l[j] = have ? s16 : 0.f;
-    }
-    if constexpr (KINDS) {
-      bool fin = true;
-#pragma unroll
-      for (int k = 0; k < 8; ++k) fin = fin && fabsf(v[k]) <= 3.40282347e38f;
-      finite = !have || fin;
-    }
-  }
-  {
-    float ss = 0.f;
-    for (uint32_t j = tid; j < (MRG ? 0u : nunit); j += NT) {
-      if constexpr (IXE) {
-        finite = stage_digits(j, ss) && finite;
-      } else if (j == tid) {  // the unit loaded above (load_unit's arithmetic)
-        float v[16];
-        if (xin) {
-#pragma unroll
-          for (int k = 0; k < 4; ++k) {
-            const float4 xv = xr[k];
-            v[4 * k] = xv.x; v[4 * k + 1] = xv.y; v[4 * k + 2] = xv.z; v[4 * k + 3] = xv.w;
-            if (NORM) {
-              const float4 wv = wr[k];
-              ss = fmaf(xv.x, xv.x, ss); ss = fmaf(xv.y, xv.y, ss);
-              ss = fmaf(xv.z, xv.z, ss); ss = fmaf(xv.w, xv.w, ss);
-              v[4 * k] *= wv.x; v[4 * k + 1] *= wv.y; v[4 * k + 2] *= wv.z; v[4 * k + 3] *= wv.w;
-            }
-          }
-        }
-        finite = put_float(j, v, xin, KINDS) && finite;
-      } else {
-        finite = stage_float(j, ss, true, KINDS) && finite;
-      }
-    }
-    if (NORM) {
-      ss = rf_wave_sum(ss);
-      if (lane == 0) wsum[wave] = ss;
-    }
-    if constexpr (KINDS) {
-      const bool bad = __ballot(!finite) != 0;
-      if (lane == 0) wbad[wave] = bad ? 1u : 0u;
-    }
-    // EPI_RESIDUAL: the residual of every row this wavefront will finish
-    // (at most PK_RES_SLOTS tasks; the launch sizes the grid for that), so
-    // the epilogue reads LDS instead of waiting on a load queued behind codes.
-    if constexpr (EPI == EPI_RESIDUAL) {
-      for (uint32_t k = 0; k < PK_RES_SLOTS; ++k) {
-        const uint32_t t = ct + k * gstride;
-        if (t >= ntask) break;
-        if (lane < (uint32_t)U) {
-          const uint32_t vr = t * U + lane;
-          float r = 0.f;
-          if (vr < a.rows_total) {
-            const PkSeg g = seg_of(vr);
-            r = g.res[vr - g.row_begin];
-          }
-          resl[wave][k][lane] = r;
-        }
-      }
-    }
-  }
-  __syncthreads();
-  // A non-finite x element (every workgroup sees the same x, so all of them
-  // agree): every row sum is then non-finite.  The reference adds the terms
-  // deq * x of a row in order (quant.rs:977-1029): NaN when a term is NaN or
-  // terms of both infinite signs occur, else the one infinity.  That depends
-  // on the terms only, not on their order, so each row's terms are classified
-  // with the reference's own weight decode instead of summed (an overflow of
-  // finite partial sums, which the reference's order could turn into NaN, is
-  // not reproduced).
-  bool bad = false;
-  if constexpr (KINDS) {
-#pragma unroll
-    for (uint32_t i = 0; i < NW; ++i) bad = bad || wbad[i] != 0u;
-  }
-  float inv = 1.f;
-  if (NORM) {
-    float tot = 0.f;
-#pragma unroll
-    for (uint32_t i = 0; i < NW; ++i) tot += wsum[i];
-    inv = 1.0f / sqrtf(tot / (float)in + a.eps);
-  }
-  if constexpr (KINDS) {
-  if (bad) {
-    if constexpr (IXE) {  // the digit layout holds no floats: stage them
-      float unused = 0.f;
-      for (uint32_t j = tid; j < nunit; j += NT) (void)stage_float(j, unused, false, false);
-      __syncthreads();
-    }
-    for (uint32_t t = blockIdx.x * NW + wave; t < ntask; t += gstride) {
-#pragma unroll
-      for (int u = 0; u < U; ++u) {
-        const uint32_t v = t * U + u;
-        if (v >= a.rows_total) break;
-        const PkSeg g = seg_of(v);
-        const uint32_t r = v - g.row_begin;
-        PkRsrc rr[F::NREG], rr2[F::NREG];
-#pragma unroll
-        for (int k = 0; k < (int)F::NREG; ++k) {
-          const uint32_t rb = (uint32_t)F::row_bytes(k, in);
-          rr[k] = __builtin_amdgcn_make_buffer_rsrc((void*)(g.reg[k] + (size_t)r * rb), 0, (int32_t)rb, PK_RSRC_WORD3);
-          if constexpr (DUAL)
-            rr2[k] = __builtin_amdgcn_make_buffer_rsrc((void*)(g.reg_up[k] + (size_t)r * rb), 0, (int32_t)rb,
-                                                       PK_RSRC_WORD3);
-        }
-        uint32_t kd = 0, kd2 = 0;
-        for (uint32_t c = 0; c < nchunk; ++c) {
-          const uint32_t b = c * 1024u + 16u * lane;
-          nv_u32x4 q, q2;
-          typename F::Meta m, m2;
-          F::fetch(q, m, rr, b);
-          if constexpr (DUAL) F::fetch(q2, m2, rr2, b);
-          if (b < crb) {
-            const float* xp = xl + c * 64u * EPL + 4u * lane;
-#pragma unroll
-            for (int i = 0; i < 4; ++i) {
-              const float4 xv = *reinterpret_cast<const float4*>(xp + 256 * i);
-              const float4 xw = UPS == 2 ? *reinterpret_cast<const float4*>(xp + 256 * (i + 4)) : xv;
-              kd |= F::kinds(LC, q[i], m, i, xv, xw);
-              if constexpr (DUAL) kd2 |= F::kinds(LC, q2[i], m2, i, xv, xw);
-            }
-          }
-        }
-        auto value = [&](uint32_t k) {
-          const bool nan = __ballot((k & 1u) != 0) != 0, pinf = __ballot((k & 2u) != 0) != 0,
-                     ninf = __ballot((k & 4u) != 0) != 0;
-          return (nan || (pinf && ninf) || !(pinf || ninf)) ? __builtin_nanf("")
-                                                             : (pinf ? __builtin_inff() : -__builtin_inff());
-        };
-        // with the fused RMSNorm, 1 / rms is 0 (or NaN) here: every row is NaN,
-        // as the reference's x / rms (inf / inf at the infinity) makes it
-        const float y0 = value(kd) * inv, y1 = DUAL ? value(kd2) * inv : 0.f;
-        if (lane == 0) {
-          const uint32_t o = v - g.row_begin;
-          if (EPI == EPI_STORE) g.y[o] = y0;
-          else if (EPI == EPI_RESIDUAL) g.y[o] = g.res[o] + y0;
-          else g.y[o] = y0 / (1.0f + expf(-y0)) * y1;
-        }
-      }
-    }
-    return;
-  }
-  }
-
-  float acc[U], acc2[U];
-#pragma unroll
-  for (int u = 0; u < U; ++u) { acc[u] = 0.f; acc2[u] = 0.f; }
-  uint32_t done = 0;  // tasks this wavefront has finished
-
-  // One step: decode LPW chunks of U rows against x (digit planes when
-  // MODE::value, else floats), then finish the rows when the task ends.
-  auto consume = [&](auto mode, const Step& B, uint32_t tt, uint32_t ss) {
-    constexpr bool DIG = IXE && decltype(mode)::value;
-#pragma unroll
-    for (int l = 0; l < LPW; ++l) {
-      // Lanes past the end of the row (a partial last chunk, or a chunk past
-      // nchunk when LPW does not divide it) decode zeros against a clamped,
-      // in-bounds slice of x and keep their sums by a select.
-      const uint32_t c = ss * LPW + l, cx = c < nchunk ? c : nchunk - 1u;
-      const bool valid = c * 1024u + 16u * lane < crb;
-      if constexpr (DIG) {
-        if constexpr (IXE) {  // only formats with idot / ifinish
-        nv_u32x4 P[PK_PLANES * UPS];
-        float2 ui[UPS];
-#pragma unroll
-        for (uint32_t h = 0; h < UPS; ++h) {
-#pragma unroll
-          for (uint32_t p = 0; p < (uint32_t)PK_PLANES; ++p)
-            P[PK_PLANES * h + p] =
-                *reinterpret_cast<const nv_u32x4*>(xdig + ((cx * UPS + h) * PK_PLANES + p) * 1024u + 16u * lane);
-          ui[h] = xinfo[(cx * 64u + lane) * UPS + h];
-        }
-#pragma unroll
-        for (int u = 0; u < U; ++u) {
-          int S[UPS][PK_PLANES] = {};
-          F::idot(LC, B.q[u][l], P, S);
-          const float f = F::ifinish(LC, B.m[u][l], S, ui);
-          acc[u] = valid ? acc[u] + f : acc[u];
-          if constexpr (DUAL) {
-            int S2[UPS][PK_PLANES] = {};
-            F::idot(LC, B.q2[u][l], P, S2);
-            const float f2 = F::ifinish(LC, B.m2[u][l], S2, ui);
-            acc2[u] = valid ? acc2[u] + f2 : acc2[u];
-          }
-        }
-        }
-      } else {
-        const float* xp = xl + cx * 64u * EPL + 4u * lane;
-        float s0[U], s1[U], t0[U], t1[U];
-#pragma unroll
-        for (int u = 0; u < U; ++u) { s0[u] = 0.f; s1[u] = 0.f; t0[u] = 0.f; t1[u] = 0.f; }
-#pragma unroll
-        for (int i = 0; i < 4; ++i) {
-          const float4 xv = *reinterpret_cast<const float4*>(xp + 256 * i);
-          float4 xw = xv;
-          if (UPS == 2) xw = *reinterpret_cast<const float4*>(xp + 256 * (i + 4));
-#pragma unroll
-          for (int u = 0; u < U; ++u) {
-            F::word(LC, B.q[u][l][i], B.m[u][l], i, xv, xw, s0[u], s1[u]);
-            if constexpr (DUAL) F::word(LC, B.q2[u][l][i], B.m2[u][l], i, xv, xw, t0[u], t1[u]);
-          }
-        }
-        const uint32_t ui = (cx * 64u + lane) * UPS;
-        const float xs0 = xsum_l[ui], xs1 = UPS == 2 ? xsum_l[ui + 1u] : 0.f;
-#pragma unroll
-        for (int u = 0; u < U; ++u) {
-          const float f = F::finish(LC, B.m[u][l], s0[u], s1[u], xs0, xs1);
-          acc[u] = valid ? acc[u] + f : acc[u];
-          if constexpr (DUAL) {
-            const float f2 = F::finish(LC, B.m2[u][l], t0[u], t1[u], xs0, xs1);
-            acc2[u] = valid ? acc2[u] + f2 : acc2[u];
-          }
-        }
-      }
-    }
-    if (ss + 1u == nstep) {  // the task's rows are complete
-#pragma unroll
-      for (int u = 0; u < U; ++u) {
-        const float v = rf_wave_sum(acc[u]) * inv;
-        const float v2 = DUAL ? rf_wave_sum(acc2[u]) * inv : 0.f;
-        acc[u] = 0.f;
-        acc2[u] = 0.f;
-        const uint32_t vr = tt * U + u;  // wave-uniform
-        if (lane == (uint32_t)u && vr < a.rows_total) {
-          const PkSeg g = seg_of(vr);
-          const uint32_t o = vr - g.row_begin;
-          if (EPI == EPI_STORE) {
-            g.y[o] = v;
-          } else if (EPI == EPI_RESIDUAL) {
-            // add_reference (compute.rs:321-327); the launch keeps done < PK_RES_SLOTS
-            g.y[o] = (done < PK_RES_SLOTS ? resl[wave][done][u] : g.res[o]) + v;
-          } else {
-            g.y[o] = v / (1.0f + expf(-v)) * v2;  // silu_reference * up (compute.rs:337-350)
-          }
-        }
-      }
-      ++done;
-    }
-  };
-  // Buffer b holds step k with k % NB == b: the step NB - 1 ahead goes into
-  // the buffer freed by the previous step.  The only exit is the uniform
-  // check at the top of each step, so every buffer is consumed (its loads
-  // waited for) before it is refilled.
-  auto run = [&](auto mode) {
-    if constexpr (ALLF) {  // at most NB steps per wavefront (the launch sees to it)
-#pragma unroll
-      for (int b = 0; b < NB; ++b) {
-        if (ct >= ntask) return;
-        consume(mode, buf[b], ct, cs);
-        advance(ct, cs);
-      }
-      return;
-    }
-    for (;;) {
-#pragma unroll
-      for (int b = 0; b < NB; ++b) {
-        if (ct >= ntask) return;
-        fetch(buf[(b + NB - 1) % NB], ft, fs);
-        advance(ft, fs);
-        consume(mode, buf[b], ct, cs);
-        advance(ct, cs);
-      }
-    }
-  };
-  run(std::integral_constant<bool, IXE>());
+#include "rf_matvec_packed_body.inc"
 }
 
 // GGUF blocks -> packed layout, one thread per block (install-time only).
@@ -1013,7 +695,7 @@ __global__ __launch_bounds__(256) void pack_blocks(const uint8_t* __restrict__ r
 
 bool packed_type(uint32_t t) { return t == T_Q8_0 || t == T_Q4_0 || t == T_Q4_K || t == T_Q6_K; }
 
-static uint32_t pk_qk(uint32_t t) { return (t == T_Q4_K || t == T_Q6_K) ? 256u : 32u; }
+static uint32_t pk_qk(uint32_t t) { return (t == T_Q4_K || t == T_Q5_K || t == T_Q6_K) ? 256u : 32u; }
 static uint32_t pk_epb(uint32_t t) { return t == T_Q8_0 ? 1u : 2u; }
 
 // Region k of format t: bytes per row.
@@ -1040,17 +722,23 @@ static uint32_t pk_lds_limit() {
   return (uint32_t)cached[dev];
 }
 
-static uint64_t pk_nchunk(uint32_t t, uint64_t in_dim) { return (in_dim / pk_epb(t) + 1023) / 1024; }
+static uint64_t pk_nchunk(uint32_t t, uint64_t in_dim) { return (in_dim / pk_epb(pk_base(t)) + 1023) / 1024; }
 
-PkPlan plan_packed(uint32_t t, uint64_t in_dim) {
+static PkPlan pk_plan(uint32_t t, uint64_t in_dim) {
   PkPlan p{};
-  if (!packed_type(t) || in_dim == 0 || in_dim % pk_qk(t) != 0 || in_dim > (1u << 24)) return p;
+  if (in_dim == 0 || in_dim % pk_qk(t) != 0 || in_dim > (1u << 24)) return p;
   const uint64_t nchunk = pk_nchunk(t, in_dim), ups = pk_epb(t), epl = 16 * ups;
   const uint64_t lds = (nchunk * 64 * epl + nchunk * 64 * ups) * 4;
-  if (lds + PK_STATIC_LDS > pk_lds_limit()) return p;
+  if (lds + PK_STATIC_LDS > 65536 && lds + PK_STATIC_LDS > pk_lds_limit()) return p;  // every device has 64 KiB
   p.ok = true;
   p.lds_bytes = (uint32_t)lds;
   return p;
+}
+
+PkPlan plan_packed(uint32_t t, uint64_t in_dim) { return packed_type(t) ? pk_plan(t, in_dim) : PkPlan{}; }
+
+PkPlan plan_gguf(uint32_t t, uint64_t in_dim) {
+  return packed_type(t) || t == T_Q5_0 || t == T_Q5_K ? pk_plan(t, in_dim) : PkPlan{};
 }
 
 static int pk_cu_count() {
@@ -1098,15 +786,24 @@ static int pk_occupancy(PkOccCache& c, const void* kern, int nt, uint32_t lds, h
 // Name of the matvec_packed instance the calling thread launched (or, in a
 // planning pass, would launch) last, spelled as the profiler's kernel trace
 // spells it, so that a measurement can be matched to the kernel that ran.
-static thread_local char t_last_kernel[128];
+// Each instance's name is made once (a snprintf per launch cost an eager call
+// 0.4 us).
+static thread_local const char* t_last_kernel = "";
 template <uint32_t T, int EPI, bool NORM, int U, int LPW, int NB, int NT, bool IX, bool ALLF, bool MRG>
 static void note_kernel() {
-  auto b = [](bool v) { return v ? "true" : "false"; };
-  snprintf(t_last_kernel, sizeof t_last_kernel, "void rf::matvec_packed<%uu, %d, %s, %d, %d, %d, %d, %s, %s, %s>(rf::PkArgs)",
-           T, EPI, b(NORM), U, LPW, NB, NT, b(IX), b(ALLF), b(MRG));
+  struct Name {
+    char s[128];
+    Name() {
+      auto b = [](bool v) { return v ? "true" : "false"; };
+      snprintf(s, sizeof s, "void rf::matvec_packed<%uu, %d, %s, %d, %d, %d, %d, %s, %s, %s>(rf::PkArgs)", T, EPI, b(NORM),
+               U, LPW, NB, NT, b(IX), b(ALLF), b(MRG));
+    }
+  };
+  static const Name name;
+  t_last_kernel = name.s;
 }
 const char* last_packed_kernel() { return t_last_kernel; }
-void clear_last_packed_kernel() { t_last_kernel[0] = 0; }
+void clear_last_packed_kernel() { t_last_kernel = ""; }
 
 // x as digit planes on the launches with >= 24 KiB of codes per wavefront
 // (1), on every Q8_0 / Q4_0 launch whose LDS holds them (2), or float x
@@ -1153,11 +850,19 @@ static uint64_t pk_grid(uint64_t tasks, uint64_t nw, int occ, int epi, uint64_t 
   return grid;
 }
 
+// The float-x kernel of a launch and its arguments: matvec_gguf for GGUF bytes.
+template <uint32_t T> using PkKernelArgs = std::conditional_t<(T & PK_GGUF) != 0, PkPlainArgs, PkArgs>;
+template <uint32_t T, int EPI, bool NORM, int LPW, int NB, int NT, bool ALLF>
+static constexpr auto pk_kernel() {
+  if constexpr ((T & PK_GGUF) != 0) return matvec_gguf<T, LPW, NB, NT, ALLF>;
+  else return matvec_packed<T, EPI, NORM, 1, LPW, NB, NT, false, ALLF>;
+}
+
 template <uint32_t T, int EPI, bool NORM, int LPW, int NB, int NT>
-static hipError_t launch_pk(const PkArgs& a, uint32_t lds, hipStream_t st) {
+static hipError_t launch_pk(const PkKernelArgs<T>& a, uint32_t lds, hipStream_t st) {
   constexpr int U = 1;
   static PkOccCache cache, cache_ix;  // one per kernel variant
-  auto kern = matvec_packed<T, EPI, NORM, U, LPW, NB, NT, false>;
+  auto kern = pk_kernel<T, EPI, NORM, LPW, NB, NT, false>();
   const int occ = pk_occupancy(cache, reinterpret_cast<const void*>(kern), NT, lds, st);
   if (occ < 0) return hipErrorStreamCaptureUnsupported;
   if (occ < 1) return hipErrorInvalidConfiguration;
@@ -1185,7 +890,7 @@ static hipError_t launch_pk(const PkArgs& a, uint32_t lds, hipStream_t st) {
       return hipGetLastError();
     }
   }
-  note_kernel<T, EPI, NORM, U, LPW, NB, NT, false, false, false>();
+  if constexpr ((T & PK_GGUF) == 0) note_kernel<T, EPI, NORM, U, LPW, NB, NT, false, false, false>();
   RF_KLAUNCH(kern, dim3((uint32_t)grid), dim3(NT), lds, st, a);
   return hipGetLastError();
 }
@@ -1199,10 +904,9 @@ void set_packed_inflight(int mode) { g_inflight = mode; }
 int packed_inflight() { return g_inflight; }
 
 template <uint32_t T, int EPI, bool NORM, int LPW, int NB>
-static hipError_t launch_pk_all_nb(const PkArgs& a, uint32_t lds, uint64_t grid, hipStream_t st) {
-  note_kernel<T, EPI, NORM, 1, LPW, NB, 512, false, true, false>();
-  RF_KLAUNCH((matvec_packed<T, EPI, NORM, 1, LPW, NB, 512, false, true>), dim3((uint32_t)grid), dim3(512),
-                     lds, st, a);
+static hipError_t launch_pk_all_nb(const PkKernelArgs<T>& a, uint32_t lds, uint64_t grid, hipStream_t st) {
+  if constexpr ((T & PK_GGUF) == 0) note_kernel<T, EPI, NORM, 1, LPW, NB, 512, false, true, false>();
+  RF_KLAUNCH((pk_kernel<T, EPI, NORM, LPW, NB, 512, true>()), dim3((uint32_t)grid), dim3(512), lds, st, a);
   return hipGetLastError();
 }
 
@@ -1218,10 +922,10 @@ static hipError_t launch_pk_all_nb(const PkArgs& a, uint32_t lds, uint64_t grid,
 // 2,181 tok/s), or of 8192, eight chunks (its down projection: 6.3 against
 // 5.9 us)).  *done stays false otherwise.
 template <uint32_t T, int EPI, bool NORM, int LPW>
-static hipError_t launch_pk_all(const PkArgs& a, uint32_t lds, hipStream_t st, bool* done) {
+static hipError_t launch_pk_all(const PkKernelArgs<T>& a, uint32_t lds, hipStream_t st, bool* done) {
   *done = false;
   static PkOccCache cache;
-  auto k1 = matvec_packed<T, EPI, NORM, 1, LPW, 1, 512, false, true>;
+  auto k1 = pk_kernel<T, EPI, NORM, LPW, 1, 512, true>();
   const int occ = pk_occupancy(cache, reinterpret_cast<const void*>(k1), 512, lds, st);
   if (occ < 0) return hipErrorStreamCaptureUnsupported;
   if (occ < 1) return hipSuccess;
@@ -1312,15 +1016,15 @@ hipError_t pk_merge_supported(uint32_t t, uint64_t in_dim, uint64_t rows, uint32
 // 89.1 us; steps of 8 chunks for the 14336-wide down projection (119
 // VGPRs) from 12.5 to 14.1 us.
 template <uint32_t T, int EPI, bool NORM>
-static hipError_t launch_pk_l(const PkArgs& a, uint32_t lds, hipStream_t st) {
+static hipError_t launch_pk_l(const PkKernelArgs<T>& a, uint32_t lds, hipStream_t st) {
   const uint64_t nchunk = pk_nchunk(T, a.in_dim);
   // All-in-flight shapes: single-matrix float-x launches whose rows are 4
   // chunks (Q8_0) or 2 (Q4_0, Q4_K): in_dim 4096.
-  if constexpr (EPI != EPI_SWIGLU && T != T_Q6_K) {
+  if constexpr (EPI != EPI_SWIGLU && pk_base(T) != T_Q6_K) {
     bool done = false;
     hipError_t e = hipSuccess;
     if (g_inflight && !(PkFmt<T>::INTX && g_digits == 2)) {
-      if constexpr (T == T_Q8_0) {
+      if constexpr (pk_base(T) == T_Q8_0) {
         if (nchunk == 4) e = launch_pk_all<T, EPI, NORM, 4>(a, lds, st, &done);
       } else {
         if (nchunk == 2) e = launch_pk_all<T, EPI, NORM, 2>(a, lds, st, &done);
@@ -1329,13 +1033,13 @@ static hipError_t launch_pk_l(const PkArgs& a, uint32_t lds, hipStream_t st) {
     if (done || e != hipSuccess) return e;
   }
   uint32_t pref = EPI == EPI_SWIGLU ? 2 : 4;
-  if (T == T_Q6_K) pref /= 2;
+  if (pk_base(T) == T_Q6_K) pref /= 2;
   uint32_t lpw = 1;
   while (lpw * 2 <= pref && lpw * 2 <= nchunk) lpw *= 2;
   // Q6_K gate/up keeps 512 threads: its two streams of four regions do not
   // fit the 128 VGPRs of a 1024-thread workgroup (that form spilled to
   // scratch), so it is never instantiated.
-  constexpr bool WIDE = !(T == T_Q6_K && EPI == EPI_SWIGLU);
+  constexpr bool WIDE = !(pk_base(T) == T_Q6_K && EPI == EPI_SWIGLU);
   const bool big = WIDE && lds > 40960;
   switch (lpw * 2 + (big ? 1 : 0)) {
     case 2: return launch_pk<T, EPI, NORM, 1, 2, 512>(a, lds, st);
@@ -1347,10 +1051,10 @@ static hipError_t launch_pk_l(const PkArgs& a, uint32_t lds, hipStream_t st) {
       if constexpr (WIDE) return launch_pk<T, EPI, NORM, 2, 2, 1024>(a, lds, st);
       return hipErrorInvalidValue;
     case 8:
-      if constexpr (T != T_Q6_K && EPI != EPI_SWIGLU) return launch_pk<T, EPI, NORM, 4, 2, 512>(a, lds, st);
+      if constexpr (pk_base(T) != T_Q6_K && EPI != EPI_SWIGLU) return launch_pk<T, EPI, NORM, 4, 2, 512>(a, lds, st);
       return hipErrorInvalidValue;
     case 9:
-      if constexpr (T != T_Q6_K && EPI != EPI_SWIGLU) return launch_pk<T, EPI, NORM, 4, 2, 1024>(a, lds, st);
+      if constexpr (pk_base(T) != T_Q6_K && EPI != EPI_SWIGLU) return launch_pk<T, EPI, NORM, 4, 2, 1024>(a, lds, st);
       return hipErrorInvalidValue;
     default: return hipErrorInvalidValue;
   }
@@ -1432,6 +1136,28 @@ hipError_t launch_matvec_packed(uint32_t t, const PkSegDesc* segs, int nseg, con
     case T_Q4_K: return launch_pk_t<T_Q4_K>(a, p.lds_bytes, epi, norm_w != nullptr, st);
     case T_Q6_K: return launch_pk_t<T_Q6_K>(a, p.lds_bytes, epi, norm_w != nullptr, st);
     default: return hipErrorInvalidValue;
+  }
+}
+
+hipError_t launch_matvec_gguf(uint32_t t, const void* w, uint64_t rows, const float* x, float* y, uint64_t in_dim,
+                              const PkPlan& p, hipStream_t st) {
+  if (!p.ok || !al16(x) || rows > 0x7FFFFFFFull) return hipErrorInvalidValue;
+  if (rows == 0) return hipSuccess;
+  const PkPlainArgs a{static_cast<const uint8_t*>(w), x, y, (uint32_t)rows, (uint32_t)in_dim};
+  const bool dword = (reinterpret_cast<uintptr_t>(w) & 3u) == 0 && (in_dim / pk_qk(t)) % 2 == 0;
+  switch (t) {
+    case T_Q8_0:
+      if (dword) return launch_pk_l<T_Q8_0 | PK_GGUF | PK_DWORD, EPI_STORE, false>(a, p.lds_bytes, st);
+      return launch_pk_l<T_Q8_0 | PK_GGUF, EPI_STORE, false>(a, p.lds_bytes, st);
+    case T_Q4_0:
+      if (dword) return launch_pk_l<T_Q4_0 | PK_GGUF | PK_DWORD, EPI_STORE, false>(a, p.lds_bytes, st);
+      return launch_pk_l<T_Q4_0 | PK_GGUF, EPI_STORE, false>(a, p.lds_bytes, st);
+    case T_Q5_0: return launch_pk_l<T_Q5_0 | PK_GGUF, EPI_STORE, false>(a, p.lds_bytes, st);
+    case T_Q4_K: return launch_pk_l<T_Q4_K | PK_GGUF, EPI_STORE, false>(a, p.lds_bytes, st);
+    case T_Q5_K: return launch_pk_l<T_Q5_K | PK_GGUF, EPI_STORE, false>(a, p.lds_bytes, st);
+    default:
+      if (dword) return launch_pk_l<T_Q6_K | PK_GGUF | PK_DWORD, EPI_STORE, false>(a, p.lds_bytes, st);
+      return launch_pk_l<T_Q6_K | PK_GGUF, EPI_STORE, false>(a, p.lds_bytes, st);
   }
 }
 

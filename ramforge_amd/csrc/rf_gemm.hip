@@ -6,15 +6,27 @@
 // times x in three bf16 pieces on the matrix cores, the block scale applied in
 // f32 to each block's partial sum.  What differs is who does what how often:
 //   * x is split once per launch (mm_split_x) into planes laid out as the
-//     MFMA's A operand reads them: [k / 16][token tile][piece][lane][8], one
-//     contiguous KiB per wavefront load, straight to registers.  The pieces
+//     MFMA's A operand reads them: [32-element block][half][token tile][piece]
+//     [lane][8], one contiguous KiB per wavefront load, straight to registers.  The pieces
 //     are truncations (8 significant bits each), so hi + mid + lo is x exactly.
 //   * a workgroup of four wavefronts decodes 256 weight rows of a 64-element
 //     stage into LDS once, as bf16 in B operand order, for all its tokens
 //     (WM wavefronts of 32 tokens).
-//   * v_mfma_f32_32x32x16_bf16: a 32 x 32 tile takes six for a block of 32
-//     elements (192 matrix cycles) and 16 scale FMAs (64 VALU cycles).
-//   * the x planes and the scales of odd blocks carry a minus sign: the matrix
+//   * a 32 x 32 tile takes 192 matrix cycles for a block of 32 elements and 16
+//     scale FMAs (64 VALU cycles).  Q8_0 and Q4_0 use v_mfma_f32_16x16x32_bf16:
+//     two short chains per 16-row tile leave the registers for a pipeline in
+//     which the scale FMAs, the LDS reads and the decode run under the MFMAs
+//     (stage_k32).  Left to the compiler the chain, its FMAs and the next LDS
+//     read took turns: 46% of the cycles with the matrix cores busy.  Q8_0 on
+//     one chip, 32 x 32 x 16 against this: 28672 x 4096, 512 tokens 381 and
+//     353 us, 128 tokens 117 and 105; 6144 x 4096, 96 tokens 44.0 and 39.4;
+//     4096 x 14336, 512 tokens 197 and 182.
+//   * Q4_K and Q6_K stay with v_mfma_f32_32x32x16_bf16: Q6_K has a scale per 16
+//     elements, half a 16 x 16 x 32 operand, and Q4_K's mins want the
+//     32 x 32 x 2 f32 form (as 16 x 16 x 4 the matrix time of two stages' mins
+//     is the same and the registers spill: 28672 x 4096, 512 tokens 390 us
+//     either way, 4096 x 14336, 96 tokens 67 and 72).
+//   * the x planes and the scales of odd 32-element blocks carry a minus sign: the matrix
 //     cores' chained sums round towards minus infinity, which would add up
 //     over a row (a mean error of 0.7 of the rms one at K = 14336; with the
 //     signs 0.03) and so takes itself off.
@@ -26,6 +38,7 @@
 namespace rf {
 
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
+typedef float f32x4 __attribute__((ext_vector_type(4)));
 typedef float f32x16 __attribute__((ext_vector_type(16)));
 typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
 
@@ -55,33 +68,50 @@ __device__ __forceinline__ uint2 gt_bf16(uint32_t w) {
   return make_uint2(__builtin_amdgcn_perm(b, a, 0x07060302u), __builtin_amdgcn_perm(d, c, 0x07060302u));
 }
 
-// LDS byte of piece (row, 16-element quarter kq, 8-element half h) of a stage:
-// fragment (row / 32, kq), slot 32 h + row % 32 with its low bits permuted by
+// LDS byte of piece (row, 16-element quarter kq, 8-element half h) of a stage.
+// K32 (operands of 16 rows x 32 elements): fragment (row / 16, kq / 2), slot
+// 16 (2 (kq % 2) + h) + row % 16; otherwise (32 rows x 16 elements) fragment
+// (row / 32, kq), slot 32 h + row % 32.  The slot's low bits are permuted by
 // kq, so that the lanes of a store (two or four rows x the quarters a lane
 // holds) and of a fragment read (64 consecutive slots) hit distinct banks.
 __device__ __forceinline__ uint32_t gt_swz(uint32_t kq) { return (0x2640u >> (4u * kq)) & 0xFu; }
+template <bool K32>
 __device__ __forceinline__ uint32_t gt_slot(uint32_t row, uint32_t kq, uint32_t h) {
-  return ((row >> 5) * 4u + kq) * GT_FRAG + ((32u * h + (row & 31u)) ^ gt_swz(kq)) * 16u;
+  if constexpr (K32)
+    return ((row >> 4) * 2u + (kq >> 1)) * GT_FRAG + ((32u * (kq & 1u) + 16u * h + (row & 15u)) ^ gt_swz(kq)) * 16u;
+  else
+    return ((row >> 5) * 4u + kq) * GT_FRAG + ((32u * h + (row & 31u)) ^ gt_swz(kq)) * 16u;
 }
-// 16 codes (four words of bytes) of (row, kq)
+// 8 codes (two words of bytes) of (row, kq, h)
+template <bool K32>
+__device__ __forceinline__ void gt_put8(uint8_t* b, uint32_t row, uint32_t kq, uint32_t h, uint32_t w0, uint32_t w1) {
+  const uint2 lo = gt_bf16(w0), hi = gt_bf16(w1);
+  *reinterpret_cast<uint4*>(b + gt_slot<K32>(row, kq, h)) = make_uint4(lo.x, lo.y, hi.x, hi.y);
+}
+// 16 codes (four words of bytes) of (row, kq), 32 x 16 fragments
 __device__ __forceinline__ void gt_put16(uint8_t* b, uint32_t row, uint32_t kq, const uint32_t (&w)[4]) {
 #pragma unroll
-  for (uint32_t h = 0; h < 2; ++h) {
-    const uint2 lo = gt_bf16(w[2 * h]), hi = gt_bf16(w[2 * h + 1]);
-    *reinterpret_cast<uint4*>(b + gt_slot(row, kq, h)) = make_uint4(lo.x, lo.y, hi.x, hi.y);
-  }
+  for (uint32_t h = 0; h < 2; ++h) gt_put8<false>(b, row, kq, h, w[2 * h], w[2 * h + 1]);
 }
+__device__ __forceinline__ uint32_t gt_word(const uint4& v, int i) { return i == 0 ? v.x : i == 1 ? v.y : i == 2 ? v.z : v.w; }
 
 // One stage (64 elements of 256 rows) of a format: load() requests a thread's
 // share of the codes and row tid's scales into registers, put() decodes them
 // into LDS: codes as bf16, NS scales per row (one per block of 32 elements,
-// the second block's negated; Q6_K one per 16), Q4_K also its two mins.  Rows past the segment read as
-// zeros.
+// the second block's negated; Q6_K one per 16), Q4_K also its two mins.  K32
+// formats store one of a thread's eight 16-byte pieces at a time and its row's
+// scales apart.  Rows past the segment read as zeros.
 template <uint32_t T> struct GtW;
+
+// the low or high nibbles q of a word's bytes as signed bytes 16 (q - 8): the
+// scale takes the 16 off
+__device__ __forceinline__ uint32_t gt_top_nibbles(uint32_t w, int hi) {
+  return rf_opaque(hi ? (w & 0xF0F0F0F0u) ^ 0x80808080u : rf_top_signed(w, 4));
+}
 
 template <> struct GtW<T_Q8_0> {
   static constexpr int NREG = 2, NS = 2;
-  static constexpr bool MIN = false;
+  static constexpr bool MIN = false, K32 = true;
   uint4 c[4];
   uint32_t sc[2];
   __device__ __forceinline__ void load(const GtRsrc* rs, uint32_t row0, uint32_t rows, uint32_t s, uint32_t K,
@@ -96,12 +126,11 @@ template <> struct GtW<T_Q8_0> {
 #pragma unroll
     for (uint32_t b = 0; b < 2; ++b) sc[b] = gt_ld2(rs[1], r < rows && 2u * s + b < nb ? (r * nb + 2u * s + b) * 2u : GT_OOR);
   }
-  __device__ __forceinline__ void put(uint8_t* b, float* ds, float*, uint32_t, uint32_t tid) const {
-#pragma unroll
-    for (uint32_t i = 0; i < 4; ++i) {
-      const uint32_t w[4] = {c[i].x, c[i].y, c[i].z, c[i].w};
-      gt_put16(b, i * 64u + (tid >> 2), tid & 3u, w);
-    }
+  __device__ __forceinline__ void put(int j, uint8_t* b, uint32_t tid) const {
+    const int i = j >> 1, h = j & 1;
+    gt_put8<true>(b, i * 64u + (tid >> 2), tid & 3u, h, gt_word(c[i], 2 * h), gt_word(c[i], 2 * h + 1));
+  }
+  __device__ __forceinline__ void scales(float* ds, uint32_t tid) const {
 #pragma unroll
     for (uint32_t k = 0; k < 2; ++k) ds[k * GT_ROWS + tid] = (k ? -1.f : 1.f) * rf_half_to_float_fast(sc[k]);
   }
@@ -109,7 +138,7 @@ template <> struct GtW<T_Q8_0> {
 
 template <> struct GtW<T_Q4_0> {
   static constexpr int NREG = 2, NS = 2;
-  static constexpr bool MIN = false;
+  static constexpr bool MIN = false, K32 = true;
   uint4 c[2];
   uint32_t sc[2];
   __device__ __forceinline__ void load(const GtRsrc* rs, uint32_t row0, uint32_t rows, uint32_t s, uint32_t K,
@@ -124,21 +153,12 @@ template <> struct GtW<T_Q4_0> {
 #pragma unroll
     for (uint32_t b = 0; b < 2; ++b) sc[b] = gt_ld2(rs[1], r < rows && 2u * s + b < nb ? (r * nb + 2u * s + b) * 2u : GT_OOR);
   }
-  // codes at the top of a signed byte: 16 (q - 8), the scale takes the 16 off
-  __device__ __forceinline__ void put(uint8_t* b, float* ds, float*, uint32_t, uint32_t tid) const {
-#pragma unroll
-    for (uint32_t i = 0; i < 2; ++i) {
-      const uint32_t w[4] = {c[i].x, c[i].y, c[i].z, c[i].w};
-      uint32_t lo[4], hi[4];
-#pragma unroll
-      for (int k = 0; k < 4; ++k) {
-        lo[k] = rf_opaque(rf_top_signed(w[k], 4));
-        hi[k] = rf_opaque((w[k] & 0xF0F0F0F0u) ^ 0x80808080u);
-      }
-      const uint32_t row = i * 128u + (tid >> 1), kb = 2u * (tid & 1u);
-      gt_put16(b, row, kb, lo);
-      gt_put16(b, row, kb + 1u, hi);
-    }
+  __device__ __forceinline__ void put(int j, uint8_t* b, uint32_t tid) const {
+    const int i = j >> 2, hi = (j >> 1) & 1, h = j & 1;
+    gt_put8<true>(b, i * 128u + (tid >> 1), 2u * (tid & 1u) + hi, h, gt_top_nibbles(gt_word(c[i], 2 * h), hi),
+                  gt_top_nibbles(gt_word(c[i], 2 * h + 1), hi));
+  }
+  __device__ __forceinline__ void scales(float* ds, uint32_t tid) const {
 #pragma unroll
     for (uint32_t k = 0; k < 2; ++k) ds[k * GT_ROWS + tid] = rf_half_to_float_fast(sc[k]) * (k ? -0.0625f : 0.0625f);
   }
@@ -149,7 +169,7 @@ template <> struct GtW<T_Q4_0> {
 // and of x that meet in the accumulator are small together.
 template <> struct GtW<T_Q4_K> {
   static constexpr int NREG = 2, NS = 2;
-  static constexpr bool MIN = true;
+  static constexpr bool MIN = true, K32 = false;
   uint4 c[2];
   uint4 h;  // row tid's header: d | dmin << 16, scale bytes 0-3, 4-7, 8-11
   __device__ __forceinline__ void load(const GtRsrc* rs, uint32_t row0, uint32_t rows, uint32_t s, uint32_t K,
@@ -198,7 +218,7 @@ template <> struct GtW<T_Q4_K> {
 // 2 (2 p + i) of qh byte l.
 template <> struct GtW<T_Q6_K> {
   static constexpr int NREG = 4, NS = 4;
-  static constexpr bool MIN = false;
+  static constexpr bool MIN = false, K32 = false;
   uint4 ql[2][2], qh[2];
   uint32_t sc, d;
   __device__ __forceinline__ void load(const GtRsrc* rs, uint32_t row0, uint32_t rows, uint32_t s, uint32_t K,
@@ -257,7 +277,9 @@ struct GtArgs {
 template <uint32_t T, int WM>
 __global__ __launch_bounds__(GT_THREADS, 2) void mm_tile(GtArgs a) {
   typedef GtW<T> W;
-  constexpr int TN = 2 * WM;  // row tiles of a wavefront: 4 / WM wavefronts share 256 rows
+  constexpr int TN = 2 * WM;       // 32-row tiles of a wavefront: 4 / WM wavefronts share 256 rows
+  constexpr int RT = 2 * TN;       // the same in 16-row tiles
+  constexpr bool K32 = W::K32;     // 16 x 16 x 32 operands, else 32 x 32 x 16
   __shared__ __align__(16) uint8_t bs[2][GT_B];
   __shared__ float ds[2][W::NS * GT_ROWS];
   __shared__ float ms[2][W::MIN ? 2 * GT_ROWS : 1];
@@ -290,14 +312,71 @@ __global__ __launch_bounds__(GT_THREADS, 2) void mm_tile(GtArgs a) {
       for (uint32_t p = 0; p < 3; ++p) v[h][p] = (ap + (2u * blk + h) * kstride + p * 64u)[lane];
   };
 
+  // K32: acc[i][8 r + 4 f + e] is 16-row tile 2 i + r, token 16 f + 4 (lane / 16)
+  // + e, row lane % 16; else 32-row tile i, token 8 (e / 4) + 4 lh + e % 4, row l32
   f32x16 acc[TN];
 #pragma unroll
   for (int i = 0; i < TN; ++i)
 #pragma unroll
     for (int e = 0; e < 16; ++e) acc[i][e] = 0.f;
   const f32x16 zero = acc[0];
-  // block `blk` of the stage in buffer buf
-  auto block = [&](uint32_t buf, uint32_t blk, const bf16x8 (&v)[2][3]) {
+
+  // One stage of K32 formats, from buffer buf: 2 RT groups, (block, 16-row
+  // tile) in turn, of six MFMAs each (two token tiles x three pieces, smallest
+  // first).  Written as a pipeline, as the compiler would run each chain, its
+  // scale FMAs and the next LDS read one after the other: group g's MFMAs are
+  // interleaved with group g - 1's scale FMAs and a share of the next stage's
+  // decode, its operands were requested two groups before.
+  const uint32_t l16 = lane & 15u;
+  const uint32_t slot0 = (lane ^ gt_swz(lane >> 5)) * 16u, slot1 = (lane ^ gt_swz(2u + (lane >> 5))) * 16u;
+  auto stage_k32 = [&](uint32_t buf, bf16x8 (&a0)[2][3], bf16x8 (&a1)[2][3], uint32_t next_a, auto&& decode) {
+    bf16x8 b[3];
+    float d[4];
+    f32x4 t[2][2];
+    const uint8_t* bb = &bs[buf][wn * RT * 2u * GT_FRAG];
+    const float* db = &ds[buf][wn * RT * 16u + l16];
+    auto fetch = [&](int g) {
+      const int blk = g / RT, rt = g % RT;
+      b[g % 3] = *reinterpret_cast<const bf16x8*>(bb + (blk ? slot1 : slot0) + (rt * 2 + blk) * GT_FRAG);
+      d[g % 4] = db[blk * GT_ROWS + rt * 16];
+    };
+    auto mfma = [&](int g, int k) {  // k-th of the group: piece 2 - k / 2 of token tile k % 2
+      const int f = k & 1, p = 2 - (k >> 1);
+      f32x4& c = t[g & 1][f];
+      c = __builtin_amdgcn_mfma_f32_16x16x32_bf16(g < RT ? a0[f][p] : a1[f][p], b[g % 3],
+                                                  k < 2 ? f32x4{0.f, 0.f, 0.f, 0.f} : c, 0, 0, 0);
+    };
+    auto scale = [&](int g, int f, int e) {
+      f32x16& c = acc[g % RT / 2];
+      const int k = 8 * (g & 1) + 4 * f + e;
+      c[k] = fmaf(d[g % 4], t[g & 1][f][e], c[k]);
+    };
+    fetch(0);
+    fetch(1);
+#pragma unroll
+    for (int g = 0; g < 2 * RT; ++g) {
+      if (g + 2 < 2 * RT) fetch(g + 2);
+      mfma(g, 0);
+      mfma(g, 1);
+      __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+      for (int k = 0; k < 4; ++k) {
+        if (g > 0) {
+          scale(g - 1, k >> 1, 2 * (k & 1));
+          scale(g - 1, k >> 1, 2 * (k & 1) + 1);
+        }
+        __builtin_amdgcn_sched_barrier(0);
+        mfma(g, 2 + k);
+      }
+      if (g == RT - 1) load_a(a0, next_a);
+      if (g >= RT) decode(g - RT);
+      __builtin_amdgcn_sched_barrier(0);
+    }
+#pragma unroll
+    for (int k = 0; k < 8; ++k) scale(2 * RT - 1, k >> 2, k & 3);
+  };
+  // block `blk` of the stage in buffer buf, 32 x 32 x 16 operands
+  auto block_k16 = [&](uint32_t buf, uint32_t blk, const bf16x8 (&v)[2][3]) {
 #pragma unroll
     for (int i = 0; i < TN; ++i) {
       const uint32_t rt = wn * TN + i;
@@ -330,8 +409,7 @@ __global__ __launch_bounds__(GT_THREADS, 2) void mm_tile(GtArgs a) {
     }
   };
 
-  // lane: row l32 of each row tile, tokens 8 (e / 4) + 4 lh + e % 4.  The
-  // partials are added up in `part` every `chain` stages: chains of at most 48
+  // The partials are added up in `part` every `chain` stages: chains of at most 48
   // scale FMAs round no worse than mm_packed's split sums (relative error
   // against 64 bits at 28672 x 4096, 512 tokens: 1.3e-7; one chain of 128
   // 2.2e-7, mm_packed 1.4e-7) and cost 3% of the launch.
@@ -344,19 +422,24 @@ __global__ __launch_bounds__(GT_THREADS, 2) void mm_tile(GtArgs a) {
     for (int i = 0; i < TN; ++i) {
       // offsets past the tokens or the segment's rows write nothing; opaque,
       // so that they are computed here and not kept through the stages
-      const uint32_t r = row0 + (wn * TN + i) * 32u + l32, ld = rf_opaque(a.mtot * 4u);
-      const uint32_t o0 = r < s.rows ? 4u * lh * ld + r * 4u : GT_OOR;
+      const uint32_t r = row0 + (wn * TN + i) * 32u + (K32 ? l16 : l32), ld = rf_opaque(a.mtot * 4u);
+      const uint32_t o0 = r < s.rows ? 4u * (K32 ? lane >> 4 : lh) * ld + r * 4u : GT_OOR;
+      auto off = [&](int e) -> uint32_t {
+        if constexpr (K32)
+          return r + 16u * (e >> 3) < s.rows ? o0 + (16u * ((e >> 2) & 1) + (e & 3)) * ld + 64u * (e >> 3) : GT_OOR;
+        else
+          return r < s.rows ? o0 + (8u * (e / 4) + e % 4) * ld : GT_OOR;
+      };
       if (!first) {  // uniform
         float old[16];
 #pragma unroll
-        for (int e = 0; e < 16; ++e) old[e] = __uint_as_float(gt_ld4(pr, r < s.rows ? o0 + (8u * (e / 4) + e % 4) * ld : GT_OOR));
+        for (int e = 0; e < 16; ++e) old[e] = __uint_as_float(gt_ld4(pr, off(e)));
 #pragma unroll
         for (int e = 0; e < 16; ++e) acc[i][e] += old[e];
       }
 #pragma unroll
       for (int e = 0; e < 16; ++e) {
-        __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(acc[i][e]), pr,
-                                              r < s.rows ? o0 + (8u * (e / 4) + e % 4) * ld : GT_OOR, 0, 0);
+        __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(acc[i][e]), pr, off(e), 0, 0);
         acc[i][e] = 0.f;
       }
       __builtin_amdgcn_sched_barrier(0);
@@ -367,9 +450,18 @@ __global__ __launch_bounds__(GT_THREADS, 2) void mm_tile(GtArgs a) {
 
   W w;
   bf16x8 a0[2][3], a1[2][3];
+  auto put_all = [&](uint32_t buf, uint32_t st) {  // the stage in w
+    if constexpr (K32) {
+#pragma unroll
+      for (int j = 0; j < 8; ++j) w.put(j, bs[buf], tid);
+      w.scales(ds[buf], tid);
+    } else {
+      w.put(bs[buf], ds[buf], ms[buf], st, tid);
+    }
+  };
   w.load(rs, row0, s.rows, s0, K, tid);
   load_a(a0, 2u * s0);
-  w.put(bs[0], ds[0], ms[0], s0, tid);
+  put_all(0, s0);
   __syncthreads();
   for (uint32_t c0 = s0; c0 < s1; c0 += chain) {
     const uint32_t c1 = min(s1, c0 + chain);
@@ -377,17 +469,28 @@ __global__ __launch_bounds__(GT_THREADS, 2) void mm_tile(GtArgs a) {
       const uint32_t buf = (st - s0) & 1u, nx = min(st + 1u, s1 - 1u);  // the last stage requests itself again
       w.load(rs, row0, s.rows, nx, K, tid);
       load_a(a1, 2u * st + 1u);
-      float sx = 0.f;
-      if constexpr (W::MIN) sx = a.sums[(size_t)(2u * st + lh) * a.ntt * 32u + tt * 32u + l32];
-      block(buf, 0, a0);
-      load_a(a0, 2u * nx);
-      block(buf, 1, a1);
-      if constexpr (W::MIN) {  // plus 8 d - m times the block's sum of x: f32 products on the matrix cores
+      // the next stage's buffer: its last readers passed the barrier before
+      if constexpr (K32) {
+        stage_k32(buf, a0, a1, 2u * nx, [&](int r) {
 #pragma unroll
-        for (int i = 0; i < TN; ++i)
-          acc[i] = __builtin_amdgcn_mfma_f32_32x32x2f32(sx, ms[buf][lh * GT_ROWS + (wn * TN + i) * 32u + l32], acc[i], 0, 0, 0);
+          for (int j = r * 9 / RT; j < (r + 1) * 9 / RT; ++j) {
+            if (j < 8) w.put(j, bs[buf ^ 1u], tid);
+            else w.scales(ds[buf ^ 1u], tid);
+          }
+        });
+      } else {
+        float sx = 0.f;
+        if constexpr (W::MIN) sx = a.sums[(size_t)(2u * st + lh) * a.ntt * 32u + tt * 32u + l32];
+        block_k16(buf, 0, a0);
+        load_a(a0, 2u * nx);
+        block_k16(buf, 1, a1);
+        if constexpr (W::MIN) {  // plus 8 d - m times the block's sum of x: f32 products on the matrix cores
+#pragma unroll
+          for (int i = 0; i < TN; ++i)
+            acc[i] = __builtin_amdgcn_mfma_f32_32x32x2f32(sx, ms[buf][lh * GT_ROWS + (wn * TN + i) * 32u + l32], acc[i], 0, 0, 0);
+        }
+        put_all(buf ^ 1u, nx);
       }
-      w.put(bs[buf ^ 1u], ds[buf ^ 1u], ms[buf ^ 1u], nx, tid);  // its last readers passed the barrier before
       __syncthreads();
     }
     flush(c0 == s0);
@@ -395,20 +498,22 @@ __global__ __launch_bounds__(GT_THREADS, 2) void mm_tile(GtArgs a) {
 }
 
 // x [n][ldx] into the planes of mm_tile: one wavefront per (token tile,
-// 32-element block), odd blocks negated; tokens past n and elements past K are zeros.  SUMS: also
-// each (token, block)'s sum.  VEC: 16-byte aligned rows.
-template <bool SUMS, bool VEC>
+// 32-element block), odd blocks negated; tokens past n and elements past K are
+// zeros.  K32: fragment h is 16 tokens x 32 elements, else 32 x 16.  SUMS (not
+// K32): also each (token, block)'s sum.  VEC: 16-byte aligned rows.
+template <bool K32, bool SUMS, bool VEC>
 __global__ __launch_bounds__(256) void mm_split_x(const float* __restrict__ x, uint32_t n, uint32_t ldx, uint32_t K,
                                                   uint32_t ntt, uint32_t nblk, __bf16* __restrict__ planes,
                                                   float* __restrict__ sums) {
   const uint32_t lane = threadIdx.x & 63u, item = blockIdx.x * 4u + (threadIdx.x >> 6);
   if (item >= ntt * nblk) return;
-  const uint32_t tt = item % ntt, blk = item / ntt, t = tt * 32u + (lane & 31u);
+  const uint32_t tt = item % ntt, blk = item / ntt;
   uint4* out = reinterpret_cast<uint4*>(planes) + lane;
   float sum = 0.f;
 #pragma unroll
   for (uint32_t h = 0; h < 2; ++h) {
-    const uint32_t k = 32u * blk + 16u * h + 8u * (lane >> 5);
+    const uint32_t t = tt * 32u + (K32 ? 16u * h + (lane & 15u) : lane & 31u);
+    const uint32_t k = 32u * blk + (K32 ? 8u * (lane >> 4) : 16u * h + 8u * (lane >> 5));
     float e[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
     if (t < n && k < K) {
       const float* p = x + (size_t)t * ldx + k;
@@ -443,7 +548,7 @@ __global__ __launch_bounds__(256) void mm_split_x(const float* __restrict__ x, u
   }
   if constexpr (SUMS) {
     sum += __shfl_xor(sum, 32);
-    if (lane < 32u) sums[(size_t)blk * ntt * 32u + t] = sum;
+    if (lane < 32u) sums[(size_t)(blk * ntt + tt) * 32u + lane] = sum;
   }
 }
 
@@ -541,8 +646,9 @@ hipError_t launch_mm_tile(uint32_t t, const MmTileSeg* segs, int nseg, const flo
   const uint32_t nblk = 2 * g.nstages;
   const dim3 sg((g.ntt * nblk + 3) / 4);
   const bool vec = (reinterpret_cast<uintptr_t>(x) & 15u) == 0 && ldx % 4 == 0;
-  auto split = t == T_Q4_K ? (vec ? mm_split_x<true, true> : mm_split_x<true, false>)
-                           : (vec ? mm_split_x<false, true> : mm_split_x<false, false>);
+  auto split = t == T_Q4_K   ? (vec ? mm_split_x<false, true, true> : mm_split_x<false, true, false>)
+               : t == T_Q6_K ? (vec ? mm_split_x<false, false, true> : mm_split_x<false, false, false>)
+                             : (vec ? mm_split_x<true, false, true> : mm_split_x<true, false, false>);
   RF_KLAUNCH(split, sg, dim3(256), 0, st, x, a.n, (uint32_t)ldx, a.K, g.ntt, nblk, planes, sums);
   hipError_t e = hipGetLastError();
   if (e != hipSuccess) return e;
@@ -559,7 +665,7 @@ hipError_t launch_mm_tile(uint32_t t, const MmTileSeg* segs, int nseg, const flo
 
 hipError_t load_module_gemm() {
   hipFuncAttributes fa;
-  return hipFuncGetAttributes(&fa, reinterpret_cast<const void*>(mm_split_x<false, true>));
+  return hipFuncGetAttributes(&fa, reinterpret_cast<const void*>(mm_split_x<true, false, true>));
 }
 
 }  // namespace rf

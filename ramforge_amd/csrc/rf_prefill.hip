@@ -9,8 +9,8 @@
 // token.  Launches of more than MM_SMALL_TOKENS tokens run the tiled GEMM of
 // rf_gemm.hip: it decodes the weights and splits x once for all the tokens
 // (Q8_0, 512 tokens: 28672 x 4096 562 us in eight mm_packed launches against
-// 415, 4096 x 14336 322 against 210, 4096 x 4096 168 against 74; at 65 to 128
-// tokens the two meet, 36 against 35 us for 4096 x 4096 and 96 tokens).
+// 353, 4096 x 14336 322 against 182; up to 64 tokens mm_packed is the faster
+// one, 24 against 31 us at 6144 x 4096 and 64 tokens, 20 against 29 at 37).
 //
 // GEMM (mm_packed): Y[t][r] = sum_k W[r][k] X[t][k] on the packed layout of
 // Q8_0 / Q4_0 / Q4_K / Q6_K (rf_matvec_packed.hip).  Per 32-element step the

@@ -637,8 +637,8 @@ int32_t rf_tune_attention_kernel(int32_t mode);
  * afterwards.  Returns the value in effect (process-wide). */
 int32_t rf_tune_attention_single(int32_t positions);
 /* Batched-prefill attention: the matrix-core kernel (16-token tiles per KV
- * head, each K / V row read once per tile; G = 1, 2, 4 or 8 query heads per
- * KV head, head_dim 64 or 128) for chunks whose last token sees more than
+ * head, each K / V row read once per tile; G = 1 to 8 query heads per KV
+ * head, head_dim 64, 96 or 128) for chunks whose last token sees more than
  * 1024 positions (1, default), for every chunk (2), or never (0: the decode
  * split kernel with a token dimension, each K / V row read once per token).
  * They differ in rounding only.  Other values only query.  Returns the mode

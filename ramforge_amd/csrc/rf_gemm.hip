@@ -7,8 +7,9 @@
 // f32 to each block's partial sum.  What differs is who does what how often:
 //   * x is split once per launch (mm_split_x) into planes laid out as the
 //     MFMA's A operand reads them: [32-element block][half][token tile][piece]
-//     [lane][8], one contiguous KiB per wavefront load, straight to registers.  The pieces
-//     are truncations (8 significant bits each), so hi + mid + lo is x exactly.
+//     [lane][8], one contiguous KiB per wavefront load, straight to registers.
+//     The pieces are truncations (8 significant bits each), so hi + mid + lo is
+//     x exactly.
 //   * a workgroup of four wavefronts decodes 256 weight rows of a 64-element
 //     stage into LDS once, as bf16 in B operand order, for all its tokens
 //     (WM wavefronts of 32 tokens).
@@ -26,9 +27,9 @@
 //     32 x 32 x 2 f32 form (as 16 x 16 x 4 the matrix time of two stages' mins
 //     is the same and the registers spill: 28672 x 4096, 512 tokens 390 us
 //     either way, 4096 x 14336, 96 tokens 67 and 72).
-//   * the x planes and the scales of odd 32-element blocks carry a minus sign: the matrix
-//     cores' chained sums round towards minus infinity, which would add up
-//     over a row (a mean error of 0.7 of the rms one at K = 14336; with the
+//   * the x planes and the scales of odd 32-element blocks carry a minus sign:
+//     the matrix cores' chained sums round towards minus infinity, which would
+//     add up over a row (a mean error of 0.7 of the rms one at K = 14336; with the
 //     signs 0.03) and so takes itself off.
 // A wavefront owns 32 tokens x TN row tiles: the x planes (the larger operand,
 // three pieces) are read by one wavefront only, the weights by all from LDS.
@@ -269,7 +270,7 @@ struct GtSeg {
 struct GtArgs {
   GtSeg seg[3];
   uint32_t nseg, n, ntt, K, nstages, spp, mtot, mtiles, groups, nsplit;
-  const __bf16* planes;  // [2 nstages * 2][ntt][3][64][8]
+  const __bf16* planes;  // [2 nstages][2][ntt][3][64][8]
   const float* sums;     // [2 nstages][32 ntt] (Q4_K)
   float* part;           // [nsplit][n][mtot]
 };

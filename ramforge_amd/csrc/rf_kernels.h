@@ -75,8 +75,9 @@ void set_matvec_stream_tile(uint32_t bytes);
 uint32_t matvec_tile_bytes();
 void set_matvec_stream(bool on);
 bool matvec_stream();
-// Plain (store, no norm, one segment) Q8_0 / Q4_0 matvecs on GGUF bytes take
-// the wave-staged kernel (rf_tune_matvec_kernel 2, default).
+// Plain (store, no norm, one segment) matvecs on GGUF bytes take the kernel
+// that loads rows straight into registers, tall Q8_0 ones and F32 the
+// wave-staged ones (rf_tune_matvec_kernel 2, default).
 void set_matvec_wave(bool on);
 bool matvec_wave_on();
 // Packed Q8_0 / Q4_0 launches take x as int8 digit planes when a wavefront's

@@ -558,10 +558,9 @@ __global__ __launch_bounds__(256) void mm_split_x(const float* __restrict__ x, u
 namespace {
 constexpr uint64_t al64(uint64_t v) { return (v + 63) / 64 * 64; }
 
-// Token tiles a workgroup takes: the widest whose padding stays within a
-// quarter of the tokens' tiles.
+// Token tiles a workgroup takes (three or more tiles: launches of more than 64
+// tokens): the wider whose padding stays within a quarter of the tokens' tiles.
 uint32_t gt_wm(uint64_t ntt) {
-  if (ntt <= 2) return (uint32_t)ntt;
   return ntt % 4 == 0 || ntt % 4 == 3 || ntt > 8 ? 4u : 2u;
 }
 
@@ -602,11 +601,8 @@ uint64_t mm_tile_ws_floats(uint64_t groups, uint64_t mtot, uint64_t K, uint64_t 
 
 template <uint32_t T>
 static void launch_tile_t(const GtArgs& a, uint32_t wm, uint32_t grid, hipStream_t st) {
-  switch (wm) {
-    case 1: RF_KLAUNCH((mm_tile<T, 1>), dim3(grid), dim3(GT_THREADS), 0, st, a); break;
-    case 2: RF_KLAUNCH((mm_tile<T, 2>), dim3(grid), dim3(GT_THREADS), 0, st, a); break;
-    default: RF_KLAUNCH((mm_tile<T, 4>), dim3(grid), dim3(GT_THREADS), 0, st, a); break;
-  }
+  if (wm == 2) RF_KLAUNCH((mm_tile<T, 2>), dim3(grid), dim3(GT_THREADS), 0, st, a);
+  else RF_KLAUNCH((mm_tile<T, 4>), dim3(grid), dim3(GT_THREADS), 0, st, a);
 }
 
 hipError_t launch_mm_tile(uint32_t t, const MmTileSeg* segs, int nseg, const float* x, uint64_t ldx, uint64_t n,

@@ -1793,7 +1793,10 @@ int32_t alloc_prefill_ws(rf_model* m, uint64_t T) {
 // or of MM_SMALL_TOKENS where the budget refuses their workspace.
 int32_t ensure_prefill_ws(rf_model* m) {
   if (m->p_h) return RF_OK;
-  const uint64_t T = std::min<uint64_t>(MM_MAX_TOKENS, std::max<uint64_t>(MM_SMALL_TOKENS, (m->kv_max + 31) / 32 * 32));
+  const rf_model_config& c = m->cfg;
+  const uint64_t rows = std::max({(c.head_count + 2 * c.head_count_kv) * c.head_dim, 2 * c.feed_forward_length,
+                                  c.embedding_length});  // of a layer's tallest launch
+  const uint64_t T = std::min(mm_max_tokens(rows), std::max<uint64_t>(MM_SMALL_TOKENS, (m->kv_max + 31) / 32 * 32));
   int32_t rc = alloc_prefill_ws(m, T);
   if (rc == RF_ERR_BUDGET && T > MM_SMALL_TOKENS) rc = alloc_prefill_ws(m, MM_SMALL_TOKENS);
   return rc;

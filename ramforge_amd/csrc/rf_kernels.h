@@ -265,9 +265,9 @@ struct MmSegDesc {
 };
 bool mm_supported(uint32_t t, uint64_t in_dim);
 // Tokens of the longest launch on `rows` weight rows in all (a launch's
-// segments together): MM_MAX_TOKENS, or MM_SMALL_TOKENS where the tiled
-// kernel's 32-bit addresses would not hold.
-uint64_t mm_max_tokens(uint64_t rows);
+// segments together) of in_dim inputs: MM_MAX_TOKENS, or MM_SMALL_TOKENS where
+// its 32-bit addresses would not hold.
+uint64_t mm_max_tokens(uint64_t rows, uint64_t in_dim);
 uint64_t mm_part_floats(const uint64_t* rows, int nseg, uint64_t in_dim, uint64_t n);
 uint64_t mm_part_floats_at(const uint64_t* rows, int nseg, uint64_t in_dim, uint64_t n);
 // norm_w (EPI_RESIDUAL, one segment): also xn = RMSNorm(y) * norm_w per token

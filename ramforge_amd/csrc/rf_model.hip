@@ -1796,7 +1796,8 @@ int32_t ensure_prefill_ws(rf_model* m) {
   const rf_model_config& c = m->cfg;
   const uint64_t rows = std::max({(c.head_count + 2 * c.head_count_kv) * c.head_dim, 2 * c.feed_forward_length,
                                   c.embedding_length});  // of a layer's tallest launch
-  const uint64_t T = std::min(mm_max_tokens(rows), std::max<uint64_t>(MM_SMALL_TOKENS, (m->kv_max + 31) / 32 * 32));
+  const uint64_t inputs = std::max({c.embedding_length, c.head_count * c.head_dim, c.feed_forward_length});
+  const uint64_t T = std::min(mm_max_tokens(rows, inputs), std::max<uint64_t>(MM_SMALL_TOKENS, (m->kv_max + 31) / 32 * 32));
   int32_t rc = alloc_prefill_ws(m, T);
   if (rc == RF_ERR_BUDGET && T > MM_SMALL_TOKENS) rc = alloc_prefill_ws(m, MM_SMALL_TOKENS);
   return rc;

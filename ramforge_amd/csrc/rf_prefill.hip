@@ -805,10 +805,12 @@ static bool mm_tiled(uint64_t n) { return n > MM_SMALL_TOKENS; }
 
 // mm_tile addresses the partials of 32 tokens by 32-bit byte offsets, which
 // 2^25 rows overflow, and a launch's reduce has a thread per output, which
-// must stay below 2^32 (8.4 M rows at MM_MAX_TOKENS): taller matrices go in
-// launches of mm_packed, whose offsets are 64-bit.
-uint64_t mm_max_tokens(uint64_t rows) {
-  return rows < (1ull << 32) / MM_MAX_TOKENS ? MM_MAX_TOKENS : MM_SMALL_TOKENS;
+// must stay below 2^32 (8.4 M rows at MM_MAX_TOKENS); a launch's x stays below
+// 2^31 bytes (2^20 inputs).  Beyond, launches of mm_packed: its partials'
+// offsets are 64-bit, its x eight times shorter.
+uint64_t mm_max_tokens(uint64_t rows, uint64_t in_dim) {
+  const bool fits = rows < (1ull << 32) / MM_MAX_TOKENS && in_dim < (1ull << 31) / 4 / MM_MAX_TOKENS;
+  return fits ? MM_MAX_TOKENS : MM_SMALL_TOKENS;
 }
 
 static uint64_t mm_groups(const MmSegDesc* segs, int nseg, uint64_t rows_per_group) {
@@ -968,7 +970,7 @@ hipError_t launch_matmul_packed(uint32_t t, const MmSegDesc* segs, int nseg, con
     groups += (d.rows + rpg - 1) / rpg;
     mtot += d.rows;
   }
-  if (mtot > 0xFFFFFFFFull || groups > 0x7FFFFFFFull || n > mm_max_tokens(mtot)) return hipErrorInvalidValue;
+  if (mtot > 0xFFFFFFFFull || groups > 0x7FFFFFFFull || n > mm_max_tokens(mtot, ldx)) return hipErrorInvalidValue;
   uint32_t nsplit = 1, spp = 1, nslices = 1;
   if (!tiled) {
     mm_shape(groups, in_dim, n, &nsplit, &spp, &nslices);

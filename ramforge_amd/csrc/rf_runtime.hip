@@ -956,7 +956,7 @@ static uint64_t matmul_ws_bytes(uint64_t out_dim, uint64_t in_dim, uint64_t n_to
 
 uint64_t rf_matmul_workspace_bytes(uint64_t out_dim, uint64_t in_dim, uint64_t n_tokens) {
   if (out_dim == 0 || in_dim == 0 || n_tokens == 0) return 0;
-  return matmul_ws_bytes(out_dim, in_dim, n_tokens, mm_max_tokens(out_dim));
+  return matmul_ws_bytes(out_dim, in_dim, n_tokens, mm_max_tokens(out_dim, in_dim));
 }
 
 int32_t rf_matmul_packed(rf_ctx* ctx, uint32_t t, const void* packed, uint64_t packed_bytes, uint64_t out_dim,
@@ -987,7 +987,7 @@ int32_t rf_matmul_packed(rf_ctx* ctx, uint32_t t, const void* packed, uint64_t p
   hipStream_t st = pick_stream(ctx, s);
   // A workspace that cannot grow to the long chunks' size (fixed, being
   // captured, over the budget) may still hold the short ones'.
-  uint64_t chunk = mm_max_tokens(out_dim);
+  uint64_t chunk = mm_max_tokens(out_dim, in_dim);
   int32_t rc = ensure_workspace(ctx, ctx->mm_ws, "workspace:matmul", matmul_ws_bytes(out_dim, in_dim, n_tokens, chunk), st);
   if ((rc == RF_ERR_INVALID || rc == RF_ERR_BUDGET) && n_tokens > MM_SMALL_TOKENS && chunk > MM_SMALL_TOKENS) {
     chunk = MM_SMALL_TOKENS;

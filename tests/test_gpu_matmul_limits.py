@@ -37,6 +37,40 @@ def test_tall_matrices_take_short_launches_workspace():
     assert ws((1 << 32) // 512 - 1, 32, 512) > ws((1 << 32) // 512 - 1, 32, 64)
 
 
+def test_wide_matrices_take_short_launches_workspace():
+    """2^20 inputs: 512 tokens of x are 2^31 bytes, the most a launch takes
+    being less (host arithmetic)."""
+    from ramforge_amd import _lib
+
+    ws = _lib.load().rf_matmul_workspace_bytes
+    assert ws(8, 1 << 20, 512) == ws(8, 1 << 20, 64)
+    assert ws(8, (1 << 20) - 256, 512) > ws(8, (1 << 20) - 256, 64)
+
+
+@pytest.mark.gpu
+def test_matmul_wide(ctx):
+    """2^20 inputs and 512 tokens, each token's x the first one's times a power
+    of two: so are its results, bit for bit, and the first token's equal
+    float64's within sums of 2^20 terms in f32 (errors of 2^-24 per partial
+    sum, the partial sums growing as the square root of their length: far
+    below 2^-14 of the sum of magnitudes)."""
+    rf = _rf()
+    out_dim, in_dim, n = 8, 1 << 20, 512
+    rng = np.random.default_rng(62)
+    raw = random_matrix(Q8_0, out_dim, in_dim, rng)
+    x0 = rng.normal(0, 1, in_dim).astype(np.float32)
+    p = (np.arange(n) * 5) % 13 - 6
+    with rf.Context(0) as c:
+        dx = c.array(np.multiply.outer(np.ldexp(np.float32(1), p), x0))
+        w, y = c.array(_packed_q8_0(raw, out_dim, in_dim)), c.empty((n, out_dim))
+        rf.matmul_packed(c, Q8_0, w, (out_dim, in_dim), dx, n, y)
+        got = y.numpy()
+    wd = _weights(raw, out_dim, in_dim)
+    base = np.ldexp(got, -p[:, None])
+    assert np.array_equal(base.view(np.uint32), np.broadcast_to(base[:1], base.shape).view(np.uint32))
+    assert np.all(np.abs(base[0] - wd @ x0.astype(np.float64)) <= np.abs(wd) @ np.abs(x0) * 2.0 ** -14)
+
+
 @pytest.mark.gpu
 def test_matmul_tall(ctx):
     """2^25 + 250 rows of one 32-element block, 65 tokens, against float64:

@@ -75,6 +75,13 @@ struct Layer {
   DevTensor attn_norm, q, k, v, o, ffn_norm, gate, up, down, bq, bk, bv;
 };
 
+// The prefill workspace for chunks of up to `chunk` tokens: floats of its
+// buffers in the order of rf_model's p_h .. p_att, bytes of all (the tokens
+// behind them).
+struct PrefillWs {
+  uint64_t chunk, floats[11], part, bytes;
+};
+
 }  // namespace rf
 
 using namespace rf;
@@ -133,6 +140,7 @@ struct rf_model {
   // Batched prefill (rf_model_prefill): activations of one chunk of prompt
   // tokens and its workspaces, charged "tmp:prefill" at the first use.
   uint64_t p_chunk = 0;  // tokens of one chunk
+  std::vector<PrefillWs> p_plans;  // workspace sizes by chunk, worked out at a chunk's first use
   bool prefill_batched = false;  // rf_model_generate forwards its prompt batched
   float *p_h = nullptr, *p_xn = nullptr, *p_q = nullptr, *p_k = nullptr, *p_v = nullptr, *p_qr = nullptr;
   float *p_a = nullptr, *p_act = nullptr, *p_up = nullptr, *p_part = nullptr, *p_att = nullptr;
@@ -1732,8 +1740,9 @@ bool prefill_supported(const rf_model* m) {
   return true;
 }
 
-// The prefill workspace for chunks of up to T tokens.
-int32_t alloc_prefill_ws(rf_model* m, uint64_t T) {
+PrefillWs prefill_ws(rf_model* m, uint64_t T) {
+  for (const PrefillWs& w : m->p_plans)
+    if (w.chunk == T) return w;
   const rf_model_config& c = m->cfg;
   const uint64_t d = c.embedding_length, hd = c.head_dim, qd = c.head_count * hd;
   const uint64_t kvd = c.head_count_kv * hd, f = c.feed_forward_length;
@@ -1764,43 +1773,36 @@ int32_t alloc_prefill_ws(rf_model* m, uint64_t T) {
                                                             prefill_attention_mfma_splits(
                                                                 m->kv_max, nt, (uint32_t)c.head_count_kv)));
   const uint64_t att = recs * c.head_count * att_rec((uint32_t)hd);
-  const uint64_t sizes[] = {T * d, T * d, T * qd, T * kvd, T * kvd, T * qd, T * qd, T * f, T * f, part, att};
-  uint64_t total = 0;
-  for (uint64_t n : sizes) total += (n + 63) / 64 * 64;
-  const uint64_t bytes = total * 4 + T * 4;
+  PrefillWs w{T, {T * d, T * d, T * qd, T * kvd, T * kvd, T * qd, T * qd, T * f, T * f, part, att}, part, T * 4};
+  for (uint64_t& n : w.floats) {
+    n = (n + 63) / 64 * 64;
+    w.bytes += n * 4;
+  }
+  m->p_plans.push_back(w);
+  return w;
+}
+
+int32_t alloc_prefill_ws(rf_model* m, uint64_t T) {
+  const PrefillWs w = prefill_ws(m, T);
   int32_t rc = RF_OK;
   // a streaming model evicts cached layers to make room, as a KV growth does
   // (ensure_layer_cache_headroom, streaming_model.rs:555-572); when that is
   // not enough, the charge below reports the budget
-  if (m->streaming && (rc = make_headroom(m, bytes)) && rc != RF_ERR_BUDGET) return rc;
+  if (m->streaming && (rc = make_headroom(m, w.bytes)) && rc != RF_ERR_BUDGET) return rc;
   void* p = nullptr;
-  rc = charge_alloc(m, "tmp:prefill", bytes, &p);
+  rc = charge_alloc(m, "tmp:prefill", w.bytes, &p);
   if (rc) return rc;
   float* base = static_cast<float*>(p);
   float** dst[] = {&m->p_h,  &m->p_xn,  &m->p_q,  &m->p_k,    &m->p_v,  &m->p_qr,
                    &m->p_a,  &m->p_act, &m->p_up, &m->p_part, &m->p_att};
   for (int i = 0; i < 11; ++i) {
     *dst[i] = base;
-    base += (sizes[i] + 63) / 64 * 64;
+    base += w.floats[i];
   }
   m->p_tok = reinterpret_cast<uint32_t*>(base);
-  m->p_part_floats = part;
+  m->p_part_floats = w.part;
   m->p_chunk = T;
   return RF_OK;
-}
-
-// Chunks of MM_MAX_TOKENS tokens (fewer where the cache never holds as many),
-// or of MM_SMALL_TOKENS where the budget refuses their workspace.
-int32_t ensure_prefill_ws(rf_model* m) {
-  if (m->p_h) return RF_OK;
-  const rf_model_config& c = m->cfg;
-  const uint64_t rows = std::max({(c.head_count + 2 * c.head_count_kv) * c.head_dim, 2 * c.feed_forward_length,
-                                  c.embedding_length});  // of a layer's tallest launch
-  const uint64_t inputs = std::max({c.embedding_length, c.head_count * c.head_dim, c.feed_forward_length});
-  const uint64_t T = std::min(mm_max_tokens(rows, inputs), std::max<uint64_t>(MM_SMALL_TOKENS, (m->kv_max + 31) / 32 * 32));
-  int32_t rc = alloc_prefill_ws(m, T);
-  if (rc == RF_ERR_BUDGET && T > MM_SMALL_TOKENS) rc = alloc_prefill_ws(m, MM_SMALL_TOKENS);
-  return rc;
 }
 
 // A streaming model gives the prefill workspace back after the prompt: its
@@ -1811,8 +1813,58 @@ int32_t release_prefill_ws(rf_model* m) {
   if (rc) return rc;
   m->p_h = m->p_xn = m->p_q = m->p_k = m->p_v = m->p_qr = m->p_a = m->p_act = m->p_up = m->p_part = m->p_att = nullptr;
   m->p_tok = nullptr;
-  m->p_part_floats = 0;
+  m->p_part_floats = m->p_chunk = 0;
   return release_charge(m, "tmp:prefill");
+}
+
+// Tokens per chunk that a prompt of n tokens wants, no more than the cache ever
+// holds or a launch takes: its own token tiles where the workspace goes back
+// after it (streaming), else the next of 64, 128, 256 and 512, so that longer
+// prompts replace the workspace three times at most.
+uint64_t prefill_chunk(const rf_model* m, uint64_t n) {
+  const rf_model_config& c = m->cfg;
+  const uint64_t rows = std::max({(c.head_count + 2 * c.head_count_kv) * c.head_dim, 2 * c.feed_forward_length,
+                                  c.embedding_length});  // of a layer's tallest launch
+  const uint64_t inputs = std::max({c.embedding_length, c.head_count * c.head_dim, c.feed_forward_length});
+  const uint64_t most =
+      std::min(mm_max_tokens(rows, inputs), std::max<uint64_t>(MM_SMALL_TOKENS, (m->kv_max + 31) / 32 * 32));
+  uint64_t T = MM_SMALL_TOKENS;
+  while (T < n && T < most) T = m->streaming ? T + 32 : T * 2;
+  return std::min(T, most);
+}
+
+// Whether `bytes` more of workspace fit the budget.  A streaming model counts
+// the layers it can evict, less what the pass itself has to load: the largest
+// layer and, so that its upload overlaps, the unit after it.
+bool prefill_room(const rf_model* m, uint64_t bytes) {
+  if (!m->streaming) return vram_can_allocate(m->ctx, bytes);
+  uint64_t evictable = 0, layer = 0, unit = 0, sum = 0;
+  for (size_t u = 0; u < m->res.size(); ++u) {
+    const LayerRes& R = m->res[u];
+    if (R.state == LAYER_CACHED || R.state == LAYER_RETIRED) evictable += R.bytes;
+    sum = (u % m->upl ? sum : 0) + R.bytes;
+    layer = std::max(layer, sum);
+    unit = std::max(unit, R.bytes);
+  }
+  const uint64_t need = bytes + layer + unit;
+  return need <= evictable || vram_can_allocate(m->ctx, need - evictable);
+}
+
+// A workspace for a prompt of n tokens: the chunk it wants where that fits,
+// else shorter ones down to MM_SMALL_TOKENS, whose refusal is the caller's.  A
+// workspace that the budget or the device cannot enlarge is kept.
+int32_t ensure_prefill_ws(rf_model* m, uint64_t n) {
+  const uint64_t have = m->p_h ? m->p_chunk : 0;
+  for (uint64_t T = prefill_chunk(m, n); T > MM_SMALL_TOKENS && T > have; T = (T / 2 + 31) / 32 * 32) {
+    uint64_t held = 0;
+    if (m->p_h) held = prefill_ws(m, m->p_chunk).bytes;
+    if (!prefill_room(m, prefill_ws(m, T).bytes - held)) continue;
+    int32_t rc = m->p_h ? release_prefill_ws(m) : RF_OK;
+    if (rc) return rc;
+    rc = alloc_prefill_ws(m, T);
+    if (rc != RF_ERR_BUDGET && rc != RF_ERR_HIP) return rc;
+  }
+  return m->p_h ? RF_OK : alloc_prefill_ws(m, MM_SMALL_TOKENS);
 }
 
 // normed: p_xn already holds this layer's attention RMSNorm (the previous
@@ -1909,23 +1961,9 @@ int32_t enqueue_prefill_layer(rf_model* m, size_t li, uint64_t pos0, uint64_t nt
   return RF_OK;
 }
 
-int32_t prefill_tokens(rf_model* m, const uint32_t* tokens, uint64_t n) {
-  if (n == 0) return RF_OK;
-  if (n > m->kv_max - m->seq_len) return set_error(RF_ERR_INVALID, "KV cache full");  // seq_len <= kv_cap <= kv_max
-  for (uint64_t i = 0; i < n; ++i)
-    if (tokens[i] >= m->cfg.vocab_size)
-      return set_error(RF_ERR_INVALID, "token_id %u out of bounds for embedding with %llu rows", tokens[i],
-                       (unsigned long long)m->cfg.vocab_size);
-  int32_t rc = check_ready(m);
-  if (rc) return rc;
-  if ((rc = ensure_kv(m, m->seq_len + n))) return rc;
-  const bool batched = prefill_supported(m);
-  if (batched && (rc = ensure_prefill_ws(m)) && rc != RF_ERR_BUDGET) return rc;
-  if (!batched || rc) {  // unsupported, or a budget without room for the workspace
-    for (uint64_t i = 0; i < n; ++i)
-      if ((rc = forward_token(m, tokens[i], m->seq_len))) return rc;
-    return RF_OK;
-  }
+// The chunks of a prompt through the layers; the workspace is there.
+int32_t prefill_chunks(rf_model* m, const uint32_t* tokens, uint64_t n) {
+  int32_t rc = RF_OK;
   const rf_model_config& c = m->cfg;
   hipStream_t st = m->ctx->compute;
   const uint64_t d = c.embedding_length;
@@ -1966,7 +2004,33 @@ int32_t prefill_tokens(rf_model* m, const uint32_t* tokens, uint64_t n) {
   // the decode path continues from the last token's hidden state and position
   RF_LAUNCH(hipMemcpyAsync(m->hidden, m->p_h + (nt - 1) * d, d * 4, hipMemcpyDeviceToDevice, st), "prefill hidden");
   RF_LAUNCH(launch_set_i32(m->d_pos, (int32_t)m->seq_len, st), "prefill position");
-  return m->streaming ? release_prefill_ws(m) : RF_OK;
+  return RF_OK;
+}
+
+int32_t prefill_tokens(rf_model* m, const uint32_t* tokens, uint64_t n) {
+  if (n == 0) return RF_OK;
+  if (n > m->kv_max - m->seq_len) return set_error(RF_ERR_INVALID, "KV cache full");  // seq_len <= kv_cap <= kv_max
+  for (uint64_t i = 0; i < n; ++i)
+    if (tokens[i] >= m->cfg.vocab_size)
+      return set_error(RF_ERR_INVALID, "token_id %u out of bounds for embedding with %llu rows", tokens[i],
+                       (unsigned long long)m->cfg.vocab_size);
+  int32_t rc = check_ready(m);
+  if (rc) return rc;
+  if ((rc = ensure_kv(m, m->seq_len + n))) return rc;
+  const bool batched = prefill_supported(m);
+  if (batched && (rc = ensure_prefill_ws(m, n)) && rc != RF_ERR_BUDGET) return rc;
+  if (!batched || rc) {  // unsupported, or a budget without room for the workspace
+    for (uint64_t i = 0; i < n; ++i)
+      if ((rc = forward_token(m, tokens[i], m->seq_len))) return rc;
+    return RF_OK;
+  }
+  rc = prefill_chunks(m, tokens, n);
+  // a pass that failed gives it back as well: held, it would keep VRAM from the layers
+  if (m->streaming) {
+    const int32_t r = release_prefill_ws(m);
+    if (!rc) rc = r;
+  }
+  return rc;
 }
 
 }  // namespace

@@ -428,13 +428,16 @@ int32_t make_headroom(rf_model* m, uint64_t bytes) {
 
 constexpr uint64_t KV_GROW_CHUNK = 256;  // KvCache::GROW_CHUNK_TOKENS (kv_cache.rs:49)
 
+int32_t release_prefill_ws(rf_model* m);
+
 // Reallocate the K/V caches for `target` positions, keeping the committed
 // ones (KvCache::grow_to_with_budget, kv_cache.rs:297-356): the replacement
 // is charged "kv_cache:{k,v}:growth" while the old buffers stay charged (the
 // real peak of the copy), after streamed layers have been evicted to make
-// room for it (ensure_layer_cache_headroom); then the old buffers are freed
-// and the new charges take the old names.  On any failure the cache, its
-// charges and the captured graphs are unchanged.
+// room for it (ensure_layer_cache_headroom) or a resident model's prefill
+// workspace given back; then the old buffers are freed and the new charges
+// take the old names.  On any failure the cache, its charges and the captured
+// graphs are unchanged.
 int32_t kv_resize(rf_model* m, uint64_t target) {
   const rf_model_config& c = m->cfg;
   const uint64_t kvd = c.head_count_kv * c.head_dim, nl = c.block_count;
@@ -442,6 +445,10 @@ int32_t kv_resize(rf_model* m, uint64_t target) {
   if (m->streaming) {
     const int32_t rc = make_headroom(m, 2 * nb);
     if (rc && rc != RF_ERR_BUDGET) return rc;  // a short budget is reported by the allocation below
+  } else if (!vram_can_allocate(m->ctx, 2 * nb)) {
+    // the last prompt's workspace may be what the caches lack (the next prompt takes what is left then)
+    const int32_t rc = release_prefill_ws(m);
+    if (rc) return rc;
   }
   void *nk = nullptr, *nv = nullptr;
   int32_t rc = vram_alloc(m->ctx, "kv_cache:k:growth", nb, &nk);

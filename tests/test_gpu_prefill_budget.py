@@ -124,3 +124,31 @@ def test_failed_streaming_prompt_gives_its_workspace_back(model):
         m.reset()
         m.forward(1, 0)
         m.close()
+
+
+def test_growing_cache_takes_the_workspace_back(model):
+    """A resident model whose budget holds the K/V growth or a long prompt's
+    workspace, not both: the growth of a later step takes the workspace's
+    room, and the next prompt runs in what is left, to the hidden state of a
+    model with room to spare."""
+    rf = _rf()
+
+    def run(budget):
+        with rf.Context(0, budget) as c:
+            m = rf.GpuLlamaModel(c, CFG, CAP, kv_initial=256)
+            for name, (t, ne0, ne1, arr) in model["T"].items():
+                m.set_tensor(name, t, ne0, ne1, arr)
+            m.prefill(model["prompt"][:250])
+            held, ws = c.vram_used, c.charge(CHARGE)
+            for p in range(250, 260):  # the 257th position grows the caches
+                h = m.forward(model["prompt"][p], p, want_hidden=True)
+            grown = c.charge("kv_cache:k") + c.charge("kv_cache:v")
+            h2 = m.prefill(model["prompt"][260:400], want_hidden=True)
+            m.close()
+            return held, ws, grown, h, h2
+
+    held, ws, grown, h, h2 = run(0)
+    assert ws > grown  # so the growth fits where the workspace was
+    got = run(held + grown // 2)
+    _close(got[3], h)
+    _close(got[4], h2)

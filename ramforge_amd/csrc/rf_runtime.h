@@ -98,7 +98,8 @@ namespace rf {
 // Grow a context-owned workspace (charged as `charge`); synchronises the
 // device before releasing a smaller previous buffer.  Refused (RF_ERR_INVALID)
 // when the workspaces are fixed by rf_ctx_reserve or while `st` is being
-// captured into a graph.
+// captured into a graph, and, with the previous buffer kept, where the budget
+// or the device's free memory lacks the difference.
 int32_t ensure_workspace(rf_ctx* ctx, Workspace& ws, const char* charge, uint64_t bytes, hipStream_t st);
 // Allocate / free a ledger-charged device buffer.
 int32_t vram_alloc(rf_ctx* ctx, const std::string& charge, uint64_t bytes, void** out);

@@ -199,6 +199,21 @@ int32_t ensure_workspace(rf_ctx* ctx, Workspace& ws, const char* charge, uint64_
                      charge, (unsigned long long)bytes);
   uint64_t want = bytes < 65536 ? 65536 : bytes;
   if (ws.ptr) {
+    // A growth that the budget or the device refuses leaves the buffer: calls
+    // (and graphs) that it suffices for go on with it.
+    {
+      std::lock_guard<std::mutex> lk(ctx->mu);
+      const uint64_t avail = ctx->ledger.total() - ctx->ledger.used() + ws.bytes;
+      if (want > avail)
+        return set_error(RF_ERR_BUDGET,
+                         "insufficient memory: requested %llu bytes for '%s', but only %llu bytes available (total "
+                         "%llu, used %llu without it)",
+                         (unsigned long long)want, charge, (unsigned long long)avail,
+                         (unsigned long long)ctx->ledger.total(), (unsigned long long)(ctx->ledger.used() - ws.bytes));
+    }
+    size_t free_bytes = 0, device_bytes = 0;
+    if (hipMemGetInfo(&free_bytes, &device_bytes) == hipSuccess && want > free_bytes + ws.bytes)
+      return hip_error(hipErrorOutOfMemory, charge);
     hipError_t e = hipDeviceSynchronize();  // the old buffer may still be read by queued kernels
     if (e != hipSuccess) return hip_error(e, "hipDeviceSynchronize");
     int32_t rc = vram_release(ctx, charge);
@@ -986,10 +1001,10 @@ int32_t rf_matmul_packed(rf_ctx* ctx, uint32_t t, const void* packed, uint64_t p
                      (unsigned long long)out_dim, (unsigned long long)in_dim);
   hipStream_t st = pick_stream(ctx, s);
   // A workspace that cannot grow to the long chunks' size (fixed, being
-  // captured, over the budget) may still hold the short ones'.
+  // captured, over the budget or the device's memory) may hold the short ones'.
   uint64_t chunk = mm_max_tokens(out_dim, in_dim);
   int32_t rc = ensure_workspace(ctx, ctx->mm_ws, "workspace:matmul", matmul_ws_bytes(out_dim, in_dim, n_tokens, chunk), st);
-  if ((rc == RF_ERR_INVALID || rc == RF_ERR_BUDGET) && n_tokens > MM_SMALL_TOKENS && chunk > MM_SMALL_TOKENS) {
+  if (rc && n_tokens > MM_SMALL_TOKENS && chunk > MM_SMALL_TOKENS) {
     chunk = MM_SMALL_TOKENS;
     rc = ensure_workspace(ctx, ctx->mm_ws, "workspace:matmul", matmul_ws_bytes(out_dim, in_dim, n_tokens, chunk), st);
   }

@@ -155,3 +155,44 @@ def test_first_launch_setup_refused_inside_capture():
     root = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
     r = subprocess.run([sys.executable, "-c", _SETUP_SCRIPT, root], capture_output=True, text=True, timeout=240)
     assert r.returncode == 0 and r.stdout.strip().endswith("ok"), r.stdout + r.stderr
+
+
+def test_refused_growth_keeps_the_workspace():
+    """A budget for the 64-token launches' workspace and not for the longer
+    ones': calls of more tokens run in short launches, each with the same
+    buffer, so that a graph captured over it stays valid; the results are the
+    long launches' up to the sums' order (1e-5 of the largest output)."""
+    import ramforge_amd as rf
+    from helpers import Q8_0, pack_host, random_matrix
+
+    rng = np.random.default_rng(36)
+    rows, k, n = 700, 1024, 130
+    w = pack_host(Q8_0, random_matrix(Q8_0, rows, k, rng), rows, k)
+    x = rng.normal(0, 1, (n, k)).astype(np.float32)
+
+    def arrays(c):
+        return c.array(w), c.array(x), c.empty((n, rows))
+
+    with rf.Context(0) as c:
+        dw, dx, y = arrays(c)
+        held, short = c.vram_used, max(c.matmul_workspace_bytes(rows, k, i) for i in range(1, 65))
+        assert c.matmul_workspace_bytes(rows, k, n) > short + 65536
+        rf.matmul_packed(c, Q8_0, dw, (rows, k), dx, n, y)
+        ref = y.numpy()
+    with rf.Context(0, held + short + 65536) as c:
+        dw, dx, y = arrays(c)
+        rf.matmul_packed(c, Q8_0, dw, (rows, k), dx, n, y)
+        want, used = y.numpy(), c.vram_used
+        assert np.max(np.abs(want - ref)) <= 1e-5 * np.abs(ref).max()
+        with c.capture() as cap:
+            rf.matmul_packed(c, Q8_0, dw, (rows, k), dx, n, y)
+        for _ in range(2):
+            y.upload(np.zeros((n, rows), np.float32))
+            rf.matmul_packed(c, Q8_0, dw, (rows, k), dx, n, y)
+            assert c.vram_used == used
+            assert np.array_equal(y.numpy().view(np.uint32), want.view(np.uint32))
+            y.upload(np.zeros((n, rows), np.float32))
+            cap.graph.replay(1)
+            c.synchronize()
+            assert np.array_equal(y.numpy().view(np.uint32), want.view(np.uint32))
+        cap.graph.close()

@@ -104,7 +104,10 @@ int32_t rf_ctx_reserve(rf_ctx *ctx, uint64_t attention_bytes, uint64_t matmul_by
                        int32_t fixed);
 /* Workspace bytes of rf_attention_decode for every context of up to
  * max_positions (hist_len + 1) positions with this head shape, and of
- * rf_matmul_packed for one call of this shape (0: none needed). */
+ * rf_matmul_packed for every call of this shape with up to n_tokens tokens
+ * (0: none needed).  A matmul of more than 64 tokens whose workspace can not
+ * grow to that (fixed, being captured, refused by the budget or the device)
+ * runs in launches of 64 tokens where it holds theirs. */
 uint64_t rf_attention_workspace_bytes(uint64_t max_positions, uint32_t q_heads, uint32_t kv_heads, uint32_t head_dim);
 uint64_t rf_matmul_workspace_bytes(uint64_t out_dim, uint64_t in_dim, uint64_t n_tokens);
 rf_stream_t rf_ctx_compute_stream(rf_ctx *ctx);

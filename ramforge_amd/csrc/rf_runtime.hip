@@ -969,9 +969,29 @@ static uint64_t matmul_ws_bytes(uint64_t out_dim, uint64_t in_dim, uint64_t n_to
   return part * 4;
 }
 
+// The same for every call of up to n_tokens: a launch of fewer tokens may take
+// more splits and so more workspace (14336 x 4096: 62 MB at 128 tokens, 32 at 160).
+static uint64_t matmul_ws_bytes_upto(uint64_t out_dim, uint64_t in_dim, uint64_t n_tokens, uint64_t chunk) {
+  return mm_part_floats(&out_dim, 1, in_dim, std::min(n_tokens, chunk)) * 4;
+}
+
 uint64_t rf_matmul_workspace_bytes(uint64_t out_dim, uint64_t in_dim, uint64_t n_tokens) {
   if (out_dim == 0 || in_dim == 0 || n_tokens == 0) return 0;
-  return matmul_ws_bytes(out_dim, in_dim, n_tokens, mm_max_tokens(out_dim, in_dim));
+  return matmul_ws_bytes_upto(out_dim, in_dim, n_tokens, mm_max_tokens(out_dim, in_dim));
+}
+
+// The matmul workspace for launches of `chunk` tokens.  One that has to grow
+// grows for all shorter calls too where the budget allows, so that a shorter
+// prompt after a longer one does not replace it (and make graphs stale) again.
+static int32_t matmul_workspace(rf_ctx* ctx, uint64_t out_dim, uint64_t in_dim, uint64_t n_tokens, uint64_t chunk,
+                                hipStream_t st) {
+  const uint64_t need = matmul_ws_bytes(out_dim, in_dim, n_tokens, chunk), have = ctx->mm_ws.bytes;
+  if (have >= need) return RF_OK;
+  if (!ctx->ws_fixed && vram_can_allocate(ctx, need - have) &&
+      ensure_workspace(ctx, ctx->mm_ws, "workspace:matmul", matmul_ws_bytes_upto(out_dim, in_dim, n_tokens, chunk),
+                       st) == RF_OK)
+    return RF_OK;
+  return ensure_workspace(ctx, ctx->mm_ws, "workspace:matmul", need, st);
 }
 
 int32_t rf_matmul_packed(rf_ctx* ctx, uint32_t t, const void* packed, uint64_t packed_bytes, uint64_t out_dim,
@@ -1003,10 +1023,10 @@ int32_t rf_matmul_packed(rf_ctx* ctx, uint32_t t, const void* packed, uint64_t p
   // A workspace that cannot grow to the long chunks' size (fixed, being
   // captured, over the budget or the device's memory) may hold the short ones'.
   uint64_t chunk = mm_max_tokens(out_dim, in_dim);
-  int32_t rc = ensure_workspace(ctx, ctx->mm_ws, "workspace:matmul", matmul_ws_bytes(out_dim, in_dim, n_tokens, chunk), st);
+  int32_t rc = matmul_workspace(ctx, out_dim, in_dim, n_tokens, chunk, st);
   if (rc && n_tokens > MM_SMALL_TOKENS && chunk > MM_SMALL_TOKENS) {
     chunk = MM_SMALL_TOKENS;
-    rc = ensure_workspace(ctx, ctx->mm_ws, "workspace:matmul", matmul_ws_bytes(out_dim, in_dim, n_tokens, chunk), st);
+    rc = matmul_workspace(ctx, out_dim, in_dim, n_tokens, chunk, st);
   }
   if (rc) return rc;
   // launches of up to MM_SMALL_TOKENS tokens stage x with 16-byte loads

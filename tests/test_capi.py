@@ -74,6 +74,19 @@ def test_workspace_size_queries_without_a_gpu():
     assert lib.rf_matmul_workspace_bytes(0, 4096, 8) == 0
 
 
+def test_matmul_workspace_covers_shorter_calls():
+    """rf_matmul_workspace_bytes never shrinks with the token count, though
+    single launches do (fewer splits for more tokens): a reservation for n
+    tokens covers every call of fewer."""
+    from ramforge_amd import _lib
+
+    ws = _lib.load().rf_matmul_workspace_bytes
+    for out_dim, in_dim in ((28672, 4096), (14336, 4096), (4096, 14336), (6144, 4096), (300, 2048), (64, 256)):
+        sizes = [ws(out_dim, in_dim, n) for n in range(1, 600)]
+        assert sizes == sorted(sizes), (out_dim, in_dim)
+        assert sizes[511:] == sizes[511:512] * len(sizes[511:])
+
+
 def test_tune_switches_without_a_gpu():
     """The process-wide tune switches are host state: each returns the mode in
     effect, values outside its range only query, and the defaults are the

@@ -61,6 +61,34 @@ def test_matmul_reservation_covers_the_call():
         assert c.vram_used == used
 
 
+def test_matmul_reservation_covers_shorter_calls():
+    """A workspace fixed for 160 tokens serves 128, whose launch takes more
+    splits, with the bits of an unfixed context (the same launch, not two
+    64-token ones); without a reservation the shorter call does not replace
+    the longer one's workspace."""
+    import ramforge_amd as rf
+    from helpers import Q8_0, pack_host, random_matrix
+
+    rng = np.random.default_rng(37)
+    rows, k = 14336, 4096
+    w = pack_host(Q8_0, random_matrix(Q8_0, rows, k, rng), rows, k)
+    x = rng.normal(0, 1, (160, k)).astype(np.float32)
+    out = []
+    for first, fixed in ((128, False), (160, False), (160, True)):
+        with rf.Context(0) as c:
+            dw, dx, y = c.array(w), c.array(x), c.empty((160, rows))
+            if fixed:
+                c.reserve(matmul_bytes=c.matmul_workspace_bytes(rows, k, first), fixed=True)
+            else:
+                rf.matmul_packed(c, Q8_0, dw, (rows, k), dx, first, y)
+            used = c.vram_used
+            rf.matmul_packed(c, Q8_0, dw, (rows, k), dx, 128, y)
+            out.append(y.numpy()[:128])
+            assert c.vram_used == used
+    for got in out[1:]:
+        assert np.array_equal(got.view(np.uint32), out[0].view(np.uint32))
+
+
 def test_growth_refused_during_capture():
     import ramforge_amd as rf
 

@@ -364,7 +364,8 @@ int32_t rf_model_kv_capacity(rf_model *model, uint64_t *tokens);
  * decode step at position pos (0 for the any-shape kernel);
  * batched_prefill = 1 when rf_model_prefill (and rf_model_generate after
  * rf_model_set_prefill(1)) forwards prompts as batched GEMMs with the
- * tensors installed now, 0 when it falls back to one forward per token. */
+ * tensors installed now, 0 when it falls back to one forward per token (also
+ * when the last prompt did for want of its workspace, see rf_model_prefill). */
 int32_t rf_model_paths(rf_model *model, uint64_t pos, int32_t *split_attention, int32_t *regime,
                        int32_t *batched_prefill);
 
@@ -400,18 +401,22 @@ int32_t rf_model_decode_steps(rf_model *model, uint64_t steps);
 /* Copies the last `n` greedy tokens produced by rf_model_decode_steps. */
 int32_t rf_model_read_tokens(rf_model *model, uint32_t *out, uint64_t n);
 /* Batched prompt prefill: forwards tokens[0..n) at positions seq_len ..
- * seq_len + n - 1 in chunks of up to 512 tokens (64 where the VRAM budget
- * refuses the longer chunks' workspace, single forwards where it refuses
- * those too), each chunk through every layer
- * with the projections as rf_matmul_packed GEMMs, per-token RMSNorm, RoPE,
- * K/V cache writes and causal attention over the cache.  Same result as n
+ * seq_len + n - 1 in chunks of up to 512 tokens (fewer, down to 64, where the
+ * VRAM budget has no room for the longer chunks' workspace or, in a streaming
+ * model, for a layer beside it), each chunk through every layer with the
+ * projections as rf_matmul_packed GEMMs, per-token RMSNorm, RoPE, K/V cache
+ * writes and causal attention over the cache.  Same result as n
  * rf_model_forward calls (the reference's prompt loop, inference.rs:580-592)
  * to f32 accuracy; afterwards the model is where those calls leave it
  * (rf_model_logits, rf_model_decode_steps continue from the last token).
  * Models whose projections are not all in the packed layout (or whose
  * attention shape needs the any-shape kernel) are forwarded one token at a
- * time instead.  final_hidden as rf_model_forward, for the last token.  No
- * counterpart in the reference. */
+ * time instead.  A workspace refused at 64 tokens fails the call
+ * (RF_ERR_BUDGET); models with other than 1, 2, 4 or 8 query heads per KV head
+ * or head_dim 96 (or 256 with 8 heads) are then forwarded one token at a time
+ * as well.  A resident model keeps its workspace, grown to its longest prompt,
+ * until a K/V cache growth needs the room.  final_hidden as rf_model_forward,
+ * for the last token.  No counterpart in the reference. */
 int32_t rf_model_prefill(rf_model *model, const uint32_t *tokens, uint64_t n, float *final_hidden);
 /* rf_model_generate forwards the prompt with rf_model_prefill (1) or one
  * token at a time as the reference does (0, default). */

@@ -141,6 +141,7 @@ struct rf_model {
   // tokens and its workspaces, charged "tmp:prefill" at the first use.
   uint64_t p_chunk = 0;  // tokens of one chunk
   std::vector<PrefillWs> p_plans;  // workspace sizes by chunk, worked out at a chunk's first use
+  bool p_refused = false;        // the last prompt ran by single forwards: no room for its workspace
   bool prefill_batched = false;  // rf_model_generate forwards its prompt batched
   float *p_h = nullptr, *p_xn = nullptr, *p_q = nullptr, *p_k = nullptr, *p_v = nullptr, *p_qr = nullptr;
   float *p_a = nullptr, *p_act = nullptr, *p_up = nullptr, *p_part = nullptr, *p_att = nullptr;
@@ -1968,6 +1969,16 @@ int32_t enqueue_prefill_layer(rf_model* m, size_t li, uint64_t pos0, uint64_t nt
   return RF_OK;
 }
 
+// Whether a prompt without room for its workspace runs by single forwards.  A
+// refused workspace is the caller's error, who sizes the budget by it: single
+// forwards take ten times as long.  Group sizes other than 1, 2, 4 and 8 and
+// head_dim 96 have had single forwards only, so budgets that hold no workspace
+// are in use with them.
+bool prefill_optional(const rf_model* m) {
+  const uint64_t G = m->cfg.head_count / m->cfg.head_count_kv, hd = m->cfg.head_dim;
+  return hd == 96 || (G & (G - 1)) != 0 || !attention_per_kv((uint32_t)G, (uint32_t)hd);
+}
+
 // The chunks of a prompt through the layers; the workspace is there.
 int32_t prefill_chunks(rf_model* m, const uint32_t* tokens, uint64_t n) {
   int32_t rc = RF_OK;
@@ -2024,9 +2035,14 @@ int32_t prefill_tokens(rf_model* m, const uint32_t* tokens, uint64_t n) {
   int32_t rc = check_ready(m);
   if (rc) return rc;
   if ((rc = ensure_kv(m, m->seq_len + n))) return rc;
-  const bool batched = prefill_supported(m);
-  if (batched && (rc = ensure_prefill_ws(m, n)) && rc != RF_ERR_BUDGET) return rc;
-  if (!batched || rc) {  // unsupported, or a budget without room for the workspace
+  bool batched = prefill_supported(m);
+  m->p_refused = false;
+  if (batched && (rc = ensure_prefill_ws(m, n))) {
+    if (!prefill_optional(m) || (rc != RF_ERR_BUDGET && rc != RF_ERR_HIP)) return rc;
+    batched = false;
+    m->p_refused = true;
+  }
+  if (!batched) {
     for (uint64_t i = 0; i < n; ++i)
       if ((rc = forward_token(m, tokens[i], m->seq_len))) return rc;
     return RF_OK;
@@ -2344,7 +2360,7 @@ int32_t rf_model_paths(rf_model* m, uint64_t pos, int32_t* split_attention, int3
   if (!m || !split_attention || !regime || !batched_prefill) return set_error(RF_ERR_INVALID, "null argument");
   *split_attention = m->attn_fast ? 1 : 0;
   *regime = attn_regime(m, pos);
-  *batched_prefill = prefill_supported(m) ? 1 : 0;
+  *batched_prefill = prefill_supported(m) && !m->p_refused ? 1 : 0;
   return RF_OK;
 }
 

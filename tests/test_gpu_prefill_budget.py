@@ -152,3 +152,35 @@ def test_growing_cache_takes_the_workspace_back(model):
     got = run(held + grown // 2)
     _close(got[3], h)
     _close(got[4], h2)
+
+
+@pytest.mark.parametrize("heads,kv,hd,runs", [(4, 2, 64, False), (6, 2, 64, True), (2, 1, 96, True)])
+def test_prompt_without_room_for_any_workspace(heads, kv, hd, runs):
+    """No room for 64 tokens' workspace: the call fails and nothing is
+    forwarded, except for head groups and widths that single forwards serve;
+    those give exactly the forwards' hidden state, and paths() says so until a
+    prompt is batched again."""
+    rf = _rf()
+    cfg = dict(STREAM_CFG, context_length=256, head_count=heads, head_count_kv=kv, head_dim=hd)
+    T = _tiny_tensors(np.random.default_rng(73), cfg, ALL_Q8)
+    prompt = [int(v) for v in np.random.default_rng(74).integers(0, cfg["vocab_size"], 30)]
+    with rf.Context(0) as c:
+        m = _load_gpu(c, cfg, T, 128)
+        used = c.vram_used
+        ref = [m.forward(t, p, want_hidden=True) for p, t in enumerate(prompt)][-1]
+        m.reset()
+        m.prefill(prompt)
+        ws = c.charge(CHARGE)
+        m.close()
+    with rf.Context(0, used + ws // 2) as c:
+        m = _load_gpu(c, cfg, T, 128)
+        assert m.paths()["batched_prefill"]
+        if runs:
+            h = m.prefill(prompt, want_hidden=True)
+            assert np.array_equal(h.view(np.uint32), ref.view(np.uint32))
+            assert not m.paths()["batched_prefill"]
+        else:
+            with pytest.raises(rf.RamforgeError, match="insufficient memory"):
+                m.prefill(prompt)
+            assert m.seq_len == 0 and c.charge(CHARGE) is None
+        m.close()

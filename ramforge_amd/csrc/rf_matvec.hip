@@ -881,7 +881,12 @@ hipError_t launch_matvec_segments(uint32_t t, const MvSegDesc* segs, int nseg, c
   if (plain && wave_ok(t, in_dim, segs[0].rows, segs[0].w, x)) return launch_wave(segs[0], x, in_dim, st);
   if (plain && aligned16(x)) {
     const PkPlan g = plan_gguf(t, in_dim);
-    if (g.ok) return launch_matvec_gguf(t, segs[0].w, segs[0].rows, x, segs[0].y, in_dim, g, st);
+    if (g.ok) {
+      // Its first launch of a shape needs setup that a stream being captured
+      // refuses; the one-shot tiles and the row kernel below need none.
+      const hipError_t e = launch_matvec_gguf(t, segs[0].w, segs[0].rows, x, segs[0].y, in_dim, g, st);
+      if (e != hipErrorStreamCaptureUnsupported) return e;
+    }
   }
   MvPlan p = plan_matvec(t, in_dim, dual);
   // The tiled kernels read x and the norm weights as 16-byte vectors; other

@@ -62,3 +62,52 @@ def test_matvec_gguf_nonfinite_x_as_the_tiled_kernel(ctx, t, case):
     assert np.array_equal(out[0][~np.isnan(out[0])], out[1][~np.isnan(out[1])])
     for a in (w, dx, y):
         a.free()
+
+
+_FIRST_USE_SCRIPT = r"""
+import sys
+import numpy as np
+sys.path[:0] = [sys.argv[1], sys.argv[1] + "/tests"]
+import ramforge_amd as rf
+from helpers import GEOM, NAMES, Q4_0, Q4_K, Q5_0, Q5_K, Q6_K, Q8_0, random_matrix
+
+rng = np.random.default_rng(41)
+with rf.Context(0) as c:
+    for t in (Q8_0, Q4_0, Q5_0, Q4_K, Q5_K, Q6_K):
+        rows, in_dim = 96, 33 * 32 if GEOM[t][0] == 32 else 3 * 256
+        w = c.array(np.concatenate([np.zeros(2, np.uint8), random_matrix(t, rows, in_dim, rng)]))
+        x, y = c.array(rng.normal(0, 1, in_dim).astype(np.float32)), c.empty((rows,))
+        call = lambda: rf.matvec(c, t, w.ptr + 2, (rows, in_dim), x, y, w_bytes=w.nbytes - 2)
+        print(NAMES[t], flush=True)
+        with c.capture() as cap:  # the kernels' first launch in this process
+            call()
+        cap.graph.replay(2)
+        first = y.numpy()
+        cap.graph.close()
+        call()
+        c.synchronize()
+        eager = y.numpy()
+        assert np.max(np.abs(first - eager)) <= 1e-5 * np.abs(eager).max() and np.abs(eager).max() > 0
+        with c.capture() as cap:
+            call()
+        for _ in range(2):
+            y.upload(np.zeros(rows, np.float32))
+            cap.graph.replay(1)
+            assert np.array_equal(y.numpy().view(np.uint32), eager.view(np.uint32))
+        cap.graph.close()
+print("ok")
+"""
+
+
+def test_matvec_gguf_first_launch_inside_a_capture():
+    """Rows that are not 16-byte aligned: captured before the register kernel's
+    setup the call runs the one-shot tiles (f32 sums of a thousand terms in
+    another order: 1e-5 of the largest output), afterwards the register
+    kernel, with the eager call's bits."""
+    import os
+    import subprocess
+    import sys
+
+    root = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+    r = subprocess.run([sys.executable, "-c", _FIRST_USE_SCRIPT, root], capture_output=True, text=True, timeout=240)
+    assert r.returncode == 0 and r.stdout.strip().endswith("ok"), r.stdout + r.stderr

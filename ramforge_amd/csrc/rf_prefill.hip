@@ -899,6 +899,22 @@ static hipError_t mm_launch_shape(const MmArgs& a, dim3 grid, int ntt, bool wide
   return mm_launch_sc<T, false>(a, grid, ntt, wide, st);
 }
 
+// The one-time setup of every mm_packed instance of a type, at its first tiled
+// launch (no launch here: g_plan_only): a call of more than 64 tokens before a
+// capture is then enough for the capture to take any number, whichever kernel
+// runs them.  Not while st is being captured, where setup is refused.
+template <uint32_t T>
+static void mm_open(hipStream_t st) {
+  static bool opened = false;
+  if (opened || setup_outside_capture(st) != hipSuccess) return;
+  const bool plan = g_plan_only;
+  g_plan_only = true;
+  for (int ntt = 1; ntt <= mm_ntt(MM_SMALL_TOKENS); ++ntt)
+    for (int k = 0; k < 4; ++k) (void)mm_launch_shape<T>(MmArgs{}, dim3(1), ntt, k & 1, k & 2, st);
+  g_plan_only = plan;
+  opened = true;
+}
+
 // The wide shape unless its split fills the CUs clearly worse than the narrow
 // one (at least 95% of the narrow shape's fill), never for Q6_K.
 static bool mm_pick_wide(uint32_t t, const MmSegDesc* segs, int nseg, uint64_t in_dim, uint64_t n) {
@@ -997,6 +1013,12 @@ hipError_t launch_matmul_packed(uint32_t t, const MmSegDesc* segs, int nseg, con
   if (rope && !mm_reduce_vec4(r)) return hipErrorInvalidValue;  // before any launch
   hipError_t e;
   if (tiled) {
+    switch (t) {
+      case T_Q8_0: mm_open<T_Q8_0>(st); break;
+      case T_Q4_0: mm_open<T_Q4_0>(st); break;
+      case T_Q4_K: mm_open<T_Q4_K>(st); break;
+      default: mm_open<T_Q6_K>(st); break;
+    }
     MmTileOut o{};
     e = launch_mm_tile(t, ts, nseg, x, ldx, n, in_dim, part, part_floats, st, &o);
     r.part = o.part;

@@ -1033,9 +1033,12 @@ int32_t rf_matmul_packed(rf_ctx* ctx, uint32_t t, const void* packed, uint64_t p
   const bool aligned = (reinterpret_cast<uintptr_t>(x) & 15u) == 0 && in_dim % 4 == 0;
   const uint64_t last = n_tokens % chunk ? n_tokens % chunk : chunk, small = chunk <= MM_SMALL_TOKENS ? std::min(chunk, n_tokens)
                         : last <= MM_SMALL_TOKENS ? last : 0;
-  if (!aligned && small) {
-    rc = ensure_workspace(ctx, ctx->scratch_ws, "workspace:scratch", small * in_dim * 4, st);
-    if (rc) return rc;
+  if (!aligned) {
+    // 64 tokens' worth where it can be had, though a long launch needs none: a
+    // captured call of fewer tokens may follow
+    rc = ensure_workspace(ctx, ctx->scratch_ws, "workspace:scratch", std::min(n_tokens, MM_SMALL_TOKENS) * in_dim * 4, st);
+    if (rc && small) rc = ensure_workspace(ctx, ctx->scratch_ws, "workspace:scratch", small * in_dim * 4, st);
+    if (rc && small) return rc;
   }
   for (uint64_t off = 0; off < n_tokens; off += chunk) {
     const uint64_t nt = n_tokens - off < chunk ? n_tokens - off : chunk;

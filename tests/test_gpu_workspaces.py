@@ -185,6 +185,50 @@ def test_first_launch_setup_refused_inside_capture():
     assert r.returncode == 0 and r.stdout.strip().endswith("ok"), r.stdout + r.stderr
 
 
+_LONG_THEN_CAPTURE = r"""
+import sys
+import numpy as np
+sys.path[:0] = [sys.argv[1], sys.argv[1] + "/tests"]
+import ramforge_amd as rf
+from helpers import Q4_0, Q4_K, Q6_K, Q8_0, pack_host, random_matrix
+
+rng = np.random.default_rng(38)
+rows, k = 512, 1024
+with rf.Context(0) as c:
+    for t in (Q8_0, Q4_0, Q4_K, Q6_K):
+        w = c.array(pack_host(t, random_matrix(t, rows, k, rng), rows, k))
+        x, y = c.array(rng.normal(0, 1, 200 * k + 1).astype(np.float32)), c.empty((200, rows))
+        for xp in (x.ptr, x.ptr + 4):
+            rf.matmul_packed(c, t, w, (rows, k), xp, 200, y)
+            for n in (64, 45, 30, 5):
+                print(t, xp & 15, n, flush=True)
+                with c.capture() as cap:  # the first launches of this many tokens
+                    rf.matmul_packed(c, t, w, (rows, k), xp, n, y)
+                y.upload(np.zeros((200, rows), np.float32))
+                cap.graph.replay(2)
+                got = y.numpy()
+                cap.graph.close()
+                y.upload(np.zeros((200, rows), np.float32))
+                rf.matmul_packed(c, t, w, (rows, k), xp, n, y)
+                assert np.array_equal(got.view(np.uint32), y.numpy().view(np.uint32)) and np.any(got[n - 1])
+print("ok")
+"""
+
+
+def test_long_call_prepares_captures_of_shorter_ones():
+    """After a call of 200 tokens a capture takes any shorter call, aligned x
+    or not, though other kernels (whose setup a capture refuses) and the
+    scratch copy serve up to 64 tokens.  In a fresh process, where no shape
+    has been set up yet."""
+    import os
+    import subprocess
+    import sys
+
+    root = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+    r = subprocess.run([sys.executable, "-c", _LONG_THEN_CAPTURE, root], capture_output=True, text=True, timeout=240)
+    assert r.returncode == 0 and r.stdout.strip().endswith("ok"), r.stdout + r.stderr
+
+
 def test_refused_growth_keeps_the_workspace():
     """A budget for the 64-token launches' workspace and not for the longer
     ones': calls of more tokens run in short launches, each with the same

@@ -719,9 +719,7 @@ static hipError_t launch_wave(const MvSegDesc& s, const float* x, uint64_t in_di
   a.rows = (uint32_t)s.rows;
   a.row_bytes = (uint32_t)(in_dim / 32 * 34);
   a.region = (a.row_bytes + 16u + 15u) & ~15u;
-  switch ((a.row_bytes + 1023u) / 1024u) {
-    case 1: return launch_wave_q<1>(a, st);
-    case 2: return launch_wave_q<2>(a, st);
+  switch ((a.row_bytes + 1023u) / 1024u) {  // MVW_MIN_IN .. MVW_MAX_IN inputs: 2244 .. 4352 bytes
     case 3: return launch_wave_q<3>(a, st);
     case 4: return launch_wave_q<4>(a, st);
     default: return launch_wave_q<5>(a, st);

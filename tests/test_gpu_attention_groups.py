@@ -48,7 +48,8 @@ def test_attention_groups_equal_the_any_shape_kernel(ctx, qh, kvh, hd):
 
 
 @pytest.mark.parametrize("qh,kvh,hd,kind", [(12, 2, 128, "q4"), (6, 2, 64, "q8"), (5, 1, 96, "q8"),
-                                            (32, 2, 64, "q8"), (6, 1, 256, "q8")])
+                                            (32, 2, 64, "q8"), (6, 1, 256, "q8"), (7, 1, 64, "q8"),
+                                            (14, 2, 128, "q4")])
 def test_model_groups(ctx, orc, qh, kvh, hd, kind):
     """A prompt of 150 tokens (batched, on the matrix-core attention where it
     takes the shape and on the split kernel) and 40 teacher-forced steps past

@@ -82,6 +82,24 @@ def test_streaming_prompt_beside_its_layers(model, extra):
         m.close()
 
 
+def test_resident_prompt_in_short_chunks(model):
+    """A resident model whose budget holds a 64-token workspace and no longer
+    one: the same hidden state from 64-token chunks, and a second prompt
+    keeps the workspace."""
+    rf = _rf()
+    with rf.Context(0) as c:
+        m = _load_gpu(c, CFG, model["T"], CAP)
+        used = c.vram_used
+        m.close()
+    with rf.Context(0, used + model["short"] + 65536) as c:
+        m = _load_gpu(c, CFG, model["T"], CAP)
+        for _ in range(2):
+            _close(m.prefill(model["prompt"][:300], want_hidden=True), model["h"][0])
+            assert c.charge(CHARGE) == model["short"] and m.paths()["batched_prefill"]
+            m.reset()
+        m.close()
+
+
 @pytest.mark.parametrize("cache", [0, 1 << 30])
 def test_streaming_prompt_over_several_chunks(model, cache):
     """600 tokens: a long chunk and the rest, each layer loaded once per chunk

@@ -111,3 +111,69 @@ def test_matvec_gguf_first_launch_inside_a_capture():
     root = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
     r = subprocess.run([sys.executable, "-c", _FIRST_USE_SCRIPT, root], capture_output=True, text=True, timeout=240)
     assert r.returncode == 0 and r.stdout.strip().endswith("ok"), r.stdout + r.stderr
+
+
+def _f32(v):
+    return v.astype(np.float32).astype(np.float64)
+
+
+def _chains_of_eight(t, raw, rows, x):
+    """y = W x summed in f32 as chains of eight products per lane, scaled, over
+    a lane's steps, then over the 64 lanes in pairs: (codes [rows, blocks, lanes
+    of a block, 8], x likewise, scale [rows, blocks, lanes])."""
+    qk, size = GEOM[t]
+    b = raw.reshape(rows, -1, size)
+    nb = b.shape[1]
+
+    def half(v):  # the format's decoder: a subnormal half counts half
+        h = v.copy().view(np.float16).astype(np.float64)[..., 0]
+        return np.where(h < 2.0 ** -14, 0.5 * h, h)
+
+    if t == Q8_0:
+        q = b[..., 2:].view(np.int8).reshape(rows, nb, 4, 8).astype(np.float64)
+        xs, d = x.reshape(nb, 4, 8), np.repeat(half(b[..., :2])[..., None], 4, 2)
+    elif t == Q4_0:
+        n = b[..., 2:].reshape(rows, nb, 4, 4)
+        q = np.concatenate([n & 15, n >> 4], 3).astype(np.float64) - 8
+        xb = x.reshape(nb, 2, 4, 4)
+        xs, d = np.concatenate([xb[:, 0], xb[:, 1]], 2), np.repeat(half(b[..., :2])[..., None], 4, 2)
+    else:
+        ql, qh = b[..., :128].reshape(rows, nb, 2, 2, 32), b[..., 128:192].reshape(rows, nb, 2, 1, 32)
+        low = np.concatenate([ql & 15, ql >> 4], 3)
+        two = (qh >> np.array([0, 2, 4, 6], np.uint8)[:, None]) & 3
+        q = (low | two << 4).astype(np.float64).reshape(rows, nb, 32, 8) - 32
+        sc = np.repeat(b[..., 192:208].view(np.int8).astype(np.float64), 2, 2)
+        xs, d = x.reshape(nb, 32, 8), half(b[..., 208:210])[..., None]
+    s = np.zeros(q.shape[:3])
+    for i in range(8):
+        s = _f32(s + q[..., i] * xs[..., i])  # a fused multiply-add (53 bits hold it but for rare ties)
+    s = _f32(d * _f32(sc * s)) if t == Q6_K else _f32(d * s)
+    per = 64 // s.shape[2]  # blocks per step of 64 lanes
+    s = np.pad(s, ((0, 0), (0, -nb % per), (0, 0))).reshape(rows, -1, 64)
+    acc = np.zeros((rows, 64))
+    for k in range(s.shape[1]):
+        acc = _f32(acc + s[:, k])
+    while acc.shape[1] > 1:
+        acc = _f32(acc[:, ::2] + acc[:, 1::2])
+    return acc[:, 0]
+
+
+@pytest.mark.parametrize("t", [Q8_0, Q4_0, Q6_K])
+def test_matvec_gguf_sums_round_no_worse_than_chains_of_eight(ctx, orc, t):
+    """The rms error against float64 over 16384 rows of 1536 inputs is no larger
+    than the same products' summed in chains of eight: 4% for the sample (one
+    chain of sixteen per lane is 7 to 11% larger)."""
+    rf = _rf()
+    rng = np.random.default_rng(600 + t)
+    rows, in_dim = 16384, 1536
+    raw = random_matrix(t, rows, in_dim, rng)
+    x = rng.normal(0, 1, in_dim).astype(np.float32)
+    w, dx, y = ctx.array(raw), ctx.array(x), ctx.empty((rows,))
+    rf.matvec(ctx, t, w, (rows, in_dim), dx, y)
+    ref = orc.dequantize_rows(t, raw, in_dim, rows).astype(np.float64).reshape(rows, in_dim) @ x.astype(np.float64)
+    got, eight = (np.sqrt(np.mean((v - ref) ** 2)) for v in (y.numpy().astype(np.float64),
+                                                             _chains_of_eight(t, raw, rows, x.astype(np.float64))))
+    print(f"  {t}: rms error {got:.4e}, chains of eight {eight:.4e}, ratio {got / eight:.3f}", flush=True)
+    for a in (w, dx, y):
+        a.free()
+    assert got <= 1.04 * eight

@@ -414,8 +414,9 @@ int32_t rf_model_read_tokens(rf_model *model, uint32_t *out, uint64_t n);
  * time instead.  A workspace refused at 64 tokens fails the call
  * (RF_ERR_BUDGET); models with other than 1, 2, 4 or 8 query heads per KV head
  * or head_dim 96 (or 256 with 8 heads) are then forwarded one token at a time
- * as well.  A resident model keeps its workspace, grown to its longest prompt,
- * until a K/V cache growth needs the room.  final_hidden as rf_model_forward,
+ * as well.  A resident model keeps its workspace (the longest chunks' where the
+ * budget holds four times as much, else grown to its longest prompt) until a
+ * K/V cache growth needs the room.  final_hidden as rf_model_forward,
  * for the last token.  No counterpart in the reference. */
 int32_t rf_model_prefill(rf_model *model, const uint32_t *tokens, uint64_t n, float *final_hidden);
 /* rf_model_generate forwards the prompt with rf_model_prefill (1) or one

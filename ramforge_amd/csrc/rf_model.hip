@@ -1828,14 +1828,16 @@ int32_t release_prefill_ws(rf_model* m) {
 // Tokens per chunk that a prompt of n tokens wants, no more than the cache ever
 // holds or a launch takes: its own token tiles where the workspace goes back
 // after it (streaming), else the next of 64, 128, 256 and 512, so that longer
-// prompts replace the workspace three times at most.
-uint64_t prefill_chunk(const rf_model* m, uint64_t n) {
+// prompts replace the workspace three times at most.  A first workspace is the
+// longest at once where three quarters of the budget's rest remain.
+uint64_t prefill_chunk(rf_model* m, uint64_t n) {
   const rf_model_config& c = m->cfg;
   const uint64_t rows = std::max({(c.head_count + 2 * c.head_count_kv) * c.head_dim, 2 * c.feed_forward_length,
                                   c.embedding_length});  // of a layer's tallest launch
   const uint64_t inputs = std::max({c.embedding_length, c.head_count * c.head_dim, c.feed_forward_length});
   const uint64_t most =
       std::min(mm_max_tokens(rows, inputs), std::max<uint64_t>(MM_SMALL_TOKENS, (m->kv_max + 31) / 32 * 32));
+  if (!m->streaming && !m->p_h && vram_can_allocate(m->ctx, 4 * prefill_ws(m, most).bytes)) return most;
   uint64_t T = MM_SMALL_TOKENS;
   while (T < n && T < most) T = m->streaming ? T + 32 : T * 2;
   return std::min(T, most);

@@ -34,13 +34,20 @@ def model():
     rf = _rf()
     T = _tiny_tensors(np.random.default_rng(71), CFG, ALL_Q8)
     prompt = [int(v) for v in np.random.default_rng(72).integers(0, CFG["vocab_size"], 600)]
-    with rf.Context(0) as c:
+    with rf.Context(0) as c:  # with room to spare the first workspace is the longest
+        m = _load_gpu(c, CFG, T, CAP)
+        used = c.vram_used
+        m.prefill(prompt[:40])
+        longest = c.charge(CHARGE)
+        m.close()
+    with rf.Context(0, used + 2 * longest) as c:
         m = _load_gpu(c, CFG, T, CAP)
         m.prefill(prompt[:40])
         ws = [c.charge(CHARGE)]
         m.reset()
         h = [m.prefill(prompt[:300], want_hidden=True)]
         ws.append(c.charge(CHARGE))
+        assert ws[1] == longest
         m.reset()
         m.prefill(prompt[:20])  # a shorter prompt keeps the workspace
         assert c.charge(CHARGE) == ws[1]
@@ -60,7 +67,8 @@ def _close(got, ref):
 
 
 def test_workspace_follows_the_prompt(model):
-    """Up to 64 tokens charge 64 tokens' workspace, whatever the cache holds."""
+    """Up to 64 tokens charge 64 tokens' workspace, whatever the cache holds,
+    in a budget that the longest would fill by more than a quarter."""
     assert model["long"] > model["short"] + 2 * model["layer"] > 2 * model["layer"]
 
 
@@ -165,9 +173,11 @@ def test_growing_cache_takes_the_workspace_back(model):
             m.close()
             return held, ws, grown, h, h2
 
-    held, ws, grown, h, h2 = run(0)
+    held, ws, _, _, _ = run(0)
+    held, ws, grown, h, h2 = run(held + ws)  # not the longest workspace
     assert ws > grown  # so the growth fits where the workspace was
     got = run(held + grown // 2)
+    assert got[0] == held
     _close(got[3], h)
     _close(got[4], h2)
 
@@ -188,6 +198,11 @@ def test_prompt_without_room_for_any_workspace(heads, kv, hd, runs):
         ref = [m.forward(t, p, want_hidden=True) for p, t in enumerate(prompt)][-1]
         m.reset()
         m.prefill(prompt)
+        longest = c.charge(CHARGE)
+        m.close()
+    with rf.Context(0, used + 2 * longest) as c:
+        m = _load_gpu(c, cfg, T, 128)
+        m.prefill(prompt)
         ws = c.charge(CHARGE)
         m.close()
     with rf.Context(0, used + ws // 2) as c:
@@ -195,7 +210,7 @@ def test_prompt_without_room_for_any_workspace(heads, kv, hd, runs):
         assert m.paths()["batched_prefill"]
         if runs:
             h = m.prefill(prompt, want_hidden=True)
-            assert np.array_equal(h.view(np.uint32), ref.view(np.uint32))
+            assert (h.view(np.uint32) == ref.view(np.uint32)).all()
             assert not m.paths()["batched_prefill"]
         else:
             with pytest.raises(rf.RamforgeError, match="insufficient memory"):

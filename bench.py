@@ -474,7 +474,7 @@ def config5_bench(rf, syn, tokens: int, prompt_len: int, policy: int, persistent
         f"layer {layer / 1e6:.1f} MB, budget {budget / 2 ** 30:.0f} GiB")
     prompt = [int(t) for t in np.random.default_rng(5).integers(0, cfg["vocab_size"], prompt_len)]
     t0 = time.perf_counter()
-    m.prefill(prompt)  # batched: each streamed layer is uploaded once per 64-token chunk
+    m.prefill(prompt)  # batched: each streamed layer is uploaded once per chunk (up to 512 tokens)
     prompt_s = time.perf_counter() - t0
     pre = m.residency_stats()
     log(f"config 5: prompt {prompt_len} tokens (batched prefill) in {prompt_s:.2f} s; {pre}")
@@ -512,7 +512,7 @@ def config5_bench(rf, syn, tokens: int, prompt_len: int, policy: int, persistent
 def prefill_bench(ctx, m, cfg, rf, prompt, long_len: int) -> dict:
     """Prompt forwarding on the resident 8B-shape model: the reference's loop
     (one forward per token, inference.rs:580-592) against rf_model_prefill
-    (64-token chunks, projections as packed-weight GEMMs on the matrix cores),
+    (chunks of up to 512 tokens, projections as packed-weight GEMMs on the matrix cores),
     and a long batched prompt.  Untimed warmup prefill first (workspace, LDS
     attributes)."""
     import numpy as np
@@ -538,7 +538,7 @@ def prefill_bench(ctx, m, cfg, rf, prompt, long_len: int) -> dict:
     qd = cfg["head_count"] * cfg["head_dim"]
     kvd = cfg["head_count_kv"] * cfg["head_dim"]
     params = cfg["block_count"] * (d * (qd + 2 * kvd) + qd * d + 2 * d * f + f * d)
-    chunks = -(-long_len // 64)
+    chunks = -(-long_len // 512)  # each reads the weights once
     useful = 2.0 * long_len * params / long_s / 1e12
     out = {"prompt_tokens": len(prompt), "token_by_token_ms": round(tbt * 1e3, 2),
            "batched_ms": round(batched * 1e3, 2), "speedup": round(tbt / batched, 1),

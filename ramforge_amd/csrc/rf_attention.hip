@@ -921,7 +921,7 @@ __global__ __launch_bounds__(256) void attn_naive(AttnArgs a) {
 // contexts of more than ATT_MAX_SPLITS chunks): its single workgroup per head
 // walks K and V column by column: 512 us against 9.5 us for 12 / 2 heads, hd
 // 128, 1501 positions; the 12 / 2 head Q4_0 chat turn of 203 prompt tokens and 6
-// more (8 layers of 1536) 150 ms against 5.1 ms, its prompt batched.
+// more (8 layers of 1536) 150 ms against 3.1 ms, its prompt batched.
 bool attention_supported(uint32_t qh, uint32_t kvh, uint32_t hd, uint64_t total) {
   if (kvh == 0 || qh % kvh != 0) return false;
   if (total > (uint64_t)ATT_MAX_SPLITS * ATT_MAX_CHUNK) return false;
@@ -1056,11 +1056,17 @@ hipError_t launch_attention_naive(const AttnArgs& a, hipStream_t st) {
 }
 
 // Token batches on the matrix-core kernel (rf_tune_prefill_attention):
-// up to 8 query heads per KV head, head_dim 64, 96 or 128, cache offsets within 32 bits, and more than APF_MIN_TOTAL positions.  Timed on
-// the 8B Q8_0 prompt (32 / 8 heads, hd 128), whole prompt: 8000 tokens
-// 998 ms against 1520 ms with the split kernel, 2048 tokens 209 against 224
-// ms, but 512 tokens 49.5 against 47.8 ms: for short contexts the split
-// kernel's workgroup per token and KV head (K / V from L2) is quicker.
+// up to 8 query heads per KV head, head_dim 64, 96 or 128, cache offsets
+// within 32 bits, and more than APF_MIN_TOTAL positions: for short contexts
+// the split kernel's workgroup per token and KV head reads K / V from L2.  The
+// line was drawn with 64-token chunks (8B Q8_0, whole prompt: 8000 tokens 998
+// ms against 1520 with the split kernel, 2048 tokens 209 against 224, 512
+// tokens 49.5 against 47.8).  With 512-token chunks, us per layer, this kernel
+// against the split one: 8B Q8_0 (32 / 8 heads, hd 128) 100 tokens 267 / 256,
+// 300 567 / 563, 512 776 / 797, 1024 1592 / 1716, 2048 3340 / 4101; 12 / 2
+// heads of a 1.5B Q4_0 model 100 tokens 146 / 133, 300 210 / 213, 512 292 /
+// 288, 1024 614 / 613, 2048 1310 / 1449: between 400 and 1024 positions it would
+// now gain up to 7% or nothing.
 // Mode 2 takes the kernel at every length (tests of short prompts).
 constexpr uint64_t APF_MIN_TOTAL = 1024;
 static int g_apf = 1;
@@ -1071,10 +1077,12 @@ bool prefill_attention_mfma_supported(uint32_t qh, uint32_t kvh, uint32_t hd, ui
   const uint32_t G = qh / kvh;
   return G >= 1 && G <= 8 && (hd == 64 || hd == 96 || hd == 128) && total * kvh * hd * 4 < (1ull << 31);
 }
-// Position splits of a prefill launch on that kernel: at least enough
-// workgroups (16-token tiles x KV heads x splits) for 256 CUs, and about 256
-// positions per split past that, at most 32 and no more than chunks of
-// ATT_MIN_CHUNK positions give (att_chunk's smallest chunk).
+// Position splits of a prefill launch on that kernel: for chunks of up to 64
+// tokens at least enough workgroups (16-token tiles x KV heads x splits) for
+// 256 CUs, and about 256 positions per split past that; for longer chunks,
+// whose tiles are workgroups enough, only what fills 512 of them.  At most 32
+// and no more than chunks of ATT_MIN_CHUNK positions give (att_chunk's smallest
+// chunk).
 // Token tiles per workgroup: two for G <= 4 (the workgroup's K / V tiles
 // serve 32 tokens; 8000-token 8B prompt 965 against 997 ms with one), one
 // for larger groups (320 to 512 threads already).

@@ -17,9 +17,10 @@
 //     scale FMAs (64 VALU cycles).  Q8_0 and Q4_0 use v_mfma_f32_16x16x32_bf16:
 //     two short chains per 16-row tile leave the registers for a pipeline in
 //     which the scale FMAs, the LDS reads and the decode run under the MFMAs
-//     (stage_k32).  Left to the compiler the chain, its FMAs and the next LDS
-//     read took turns: 46% of the cycles with the matrix cores busy.  Q8_0 on
-//     one chip, 32 x 32 x 16 against this: 28672 x 4096, 512 tokens 381 and
+//     (stage_k32), where the compiler runs the chain, its FMAs and the next LDS
+//     read in turn (28672 x 4096, 512 tokens: matrix cores busy 51% of the
+//     cycles for Q8_0, 53% for Q4_0; 39% for Q6_K, left to the compiler).  Q8_0
+//     on one chip, 32 x 32 x 16 against this: 28672 x 4096, 512 tokens 381 and
 //     353 us, 128 tokens 117 and 105; 6144 x 4096, 96 tokens 44.0 and 39.4;
 //     4096 x 14336, 512 tokens 197 and 182.
 //   * Q4_K and Q6_K stay with v_mfma_f32_32x32x16_bf16: Q6_K has a scale per 16
@@ -559,7 +560,8 @@ namespace {
 constexpr uint64_t al64(uint64_t v) { return (v + 63) / 64 * 64; }
 
 // Token tiles a workgroup takes (three or more tiles: launches of more than 64
-// tokens): the wider whose padding stays within a quarter of the tokens' tiles.
+// tokens): four where that pads at most one tile, or in launches of more than
+// eight (nine to sixteen: at most three tiles of padding), else two.
 uint32_t gt_wm(uint64_t ntt) {
   return ntt % 4 == 0 || ntt % 4 == 3 || ntt > 8 ? 4u : 2u;
 }

@@ -77,3 +77,28 @@ def test_model_groups(ctx, orc, qh, kvh, hd, kind):
     finally:
         rf.tune_prefill_attention(1)
         gm.close()
+
+
+@pytest.mark.parametrize("qh,kvh,hd", [(6, 1, 256), (16, 1, 64), (7, 1, 64)])
+def test_prompt_groups_past_1024_positions(ctx, orc, qh, kvh, hd):
+    """A prompt of 1300 tokens in 512-token chunks, the last over more than one
+    1024-position chunk: per query head with the merge where no workgroup
+    takes the group (six heads of 256, sixteen), on the matrix cores for seven
+    heads; the last hidden state against the oracle's, as above."""
+    rf = _rf()
+    cfg = dict(TINY, head_count=qh, head_count_kv=kvh, head_dim=hd, embedding_length=128, block_count=1,
+               context_length=1400)
+    rng = np.random.default_rng(qh + hd)
+    T = _tiny_tensors(rng, cfg, ALL_Q8)
+    tokens = [int(v) for v in rng.integers(0, cfg["vocab_size"], 1300)]
+    om = orc.Model(cfg, T, kv_capacity=1400, threads=8)
+    for p, t in enumerate(tokens):
+        ref = om.forward(t, p)
+    om.close()
+    gm = _load_gpu(ctx, cfg, T, 1400)
+    try:
+        assert gm.paths()["batched_prefill"]
+        h = gm.prefill(tokens, want_hidden=True)
+        assert np.max(np.abs(h - ref)) <= 2e-4 * max(1.0, np.abs(ref).max())
+    finally:
+        gm.close()

@@ -148,11 +148,11 @@ def test_graph_decode_past_2048_matches_oracle(long_model):
 
 @pytest.mark.timeout(600)
 def test_prefill_1500_tokens_matches_token_by_token(long_model, orc):
-    """A 1500-token prompt through the batched prefill (64-token chunks whose
-    attention reads up to 1024 positions per chunk and merges the chunks
-    beyond) against the oracle's token-by-token forward: the last hidden
-    state and logits, then 40 graph-replayed decode steps against the
-    oracle's greedy continuation."""
+    """A 1500-token prompt through the batched prefill (512-token chunks,
+    the first two on the split attention kernel, the third, past 1024
+    positions, on the matrix-core one with its merge) against the oracle's
+    token-by-token forward: the last hidden state and logits, then 40
+    graph-replayed decode steps against the oracle's greedy continuation."""
     gm, om, _ = long_model
     assert gm.paths()["batched_prefill"], "the model's prefill fell back to one forward per token"
     rng = np.random.default_rng(2302)

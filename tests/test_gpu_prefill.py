@@ -58,8 +58,8 @@ def _check_matmul(ctx, orc, t, out_dim, in_dim, n, seed, oracle_rows=3):
                                               (300, 2048, 64), (33, 3328, 17), (1000, 5120, 100),
                                               (4096, 4096, 64), (4096, 14336, 48), (14336, 4096, 7)])
 def test_matmul_packed_matches_per_token_matvec(ctx, orc, t, out_dim, in_dim, n):
-    """Ragged token counts (1 .. 100: one to four 16-token tiles, and two
-    64-token chunks), rows not a multiple of the 128-row workgroup tile, k
+    """Ragged token counts (1 .. 64: one to four 16-token tiles; 100: the tiled
+    kernel), rows not a multiple of the 128-row workgroup tile, k
     not a multiple of the 256-element slice (Q8_0 / Q4_0), and the 8B
     projection shapes."""
     if in_dim % GEOM[t][0]:
@@ -120,7 +120,7 @@ ALL_KQ = dict(embd=Q4_K, out=Q6_K, q=Q4_K, k=Q4_K, v=Q6_K, o=Q4_K, gate=Q4_K, up
 def test_prefill_matches_token_by_token(ctx, orc, kind, history, plen):
     """Prompt of plen tokens after `history` single-token forwards: hidden
     state and logits of the last token against the oracle, then greedy
-    tokens from there.  150 and 90 tokens span several 64-token chunks; 64
+    tokens from there.  150 and 90 tokens run the tiled kernel; 64
     tokens at history 3 crosses the 64-position attention regime inside a
     chunk.  The matrix-core prefill attention runs every chunk (these
     contexts are below its default threshold); *_attn0: the decode split
@@ -304,7 +304,7 @@ def test_prefill_validation(ctx):
 
 
 def test_prefill_streaming_model(ctx, orc):
-    """Layer streaming: a batched prompt loads each layer once per 64-token
+    """Layer streaming: a batched prompt loads each layer once per
     chunk, gives the resident model's tokens and hands its workspace back
     (the layer cache may use that VRAM while decoding)."""
     cfg = dict(PF_CFG)

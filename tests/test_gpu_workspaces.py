@@ -48,7 +48,7 @@ def test_matmul_reservation_covers_the_call():
     from helpers import Q8_0, pack_host, random_matrix
 
     rng = np.random.default_rng(32)
-    rows, k, n = 512, 1024, 80  # two launches: 64 tokens and a remainder of 16
+    rows, k, n = 512, 1024, 80
     raw = random_matrix(Q8_0, rows, k, rng)
     with rf.Context(0) as c:
         w = c.array(pack_host(Q8_0, raw, rows, k))

@@ -153,6 +153,7 @@ int32_t vram_alloc(rf_ctx* ctx, const std::string& charge, uint64_t bytes, void*
   hipError_t e = hipMalloc(&p, bytes);
   if (e != hipSuccess) {
     ctx->ledger.release(charge);  // roll back the reservation
+    (void)hipGetLastError();      // callers go on with less: the next launch's check must not find it
     return hip_error(e, "hipMalloc");
   }
   ctx->buffers[charge] = p;

@@ -185,6 +185,31 @@ def test_first_launch_setup_refused_inside_capture():
     assert r.returncode == 0 and r.stdout.strip().endswith("ok"), r.stdout + r.stderr
 
 
+def test_calls_after_a_failed_device_allocation():
+    """A charge the budget allows and the device cannot hold fails without a
+    trace: the ledger is rolled back and the next calls, whose launches check
+    the runtime's last error, run."""
+    import ramforge_amd as rf
+    from helpers import Q8_0, pack_host, random_matrix
+
+    rng = np.random.default_rng(39)
+    rows, k, n = 300, 1024, 100
+    w = pack_host(Q8_0, random_matrix(Q8_0, rows, k, rng), rows, k)
+    x = rng.normal(0, 1, (n, k)).astype(np.float32)
+    out = []
+    with rf.Context(0, 1 << 50) as c:
+        dw, dx, y = c.array(w), c.array(x), c.empty((n, rows))
+        for fail in (False, True):
+            if fail:
+                used = c.vram_used
+                with pytest.raises(rf.RamforgeError, match="hipMalloc"):
+                    c.alloc(1 << 46)
+                assert c.vram_used == used
+            rf.matmul_packed(c, Q8_0, dw, (rows, k), dx, n, y)
+            out.append(y.numpy())
+    assert np.array_equal(out[0].view(np.uint32), out[1].view(np.uint32))
+
+
 _LONG_THEN_CAPTURE = r"""
 import sys
 import numpy as np

@@ -429,6 +429,7 @@ int32_t make_headroom(rf_model* m, uint64_t bytes) {
 
 constexpr uint64_t KV_GROW_CHUNK = 256;  // KvCache::GROW_CHUNK_TOKENS (kv_cache.rs:49)
 
+PrefillWs prefill_ws(rf_model* m, uint64_t T);
 int32_t release_prefill_ws(rf_model* m);
 
 // Reallocate the K/V caches for `target` positions, keeping the committed
@@ -446,10 +447,13 @@ int32_t kv_resize(rf_model* m, uint64_t target) {
   if (m->streaming) {
     const int32_t rc = make_headroom(m, 2 * nb);
     if (rc && rc != RF_ERR_BUDGET) return rc;  // a short budget is reported by the allocation below
-  } else if (!vram_can_allocate(m->ctx, 2 * nb)) {
-    // the last prompt's workspace may be what the caches lack (the next prompt takes what is left then)
-    const int32_t rc = release_prefill_ws(m);
-    if (rc) return rc;
+  } else if (m->p_h && !vram_can_allocate(m->ctx, 2 * nb)) {
+    // the last prompt's workspace where its room suffices (the next prompt takes what is left then)
+    const uint64_t held = prefill_ws(m, m->p_chunk).bytes;
+    if (2 * nb <= held || vram_can_allocate(m->ctx, 2 * nb - held)) {
+      const int32_t rc = release_prefill_ws(m);
+      if (rc) return rc;
+    }
   }
   void *nk = nullptr, *nv = nullptr;
   int32_t rc = vram_alloc(m->ctx, "kv_cache:k:growth", nb, &nk);

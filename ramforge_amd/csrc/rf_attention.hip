@@ -933,6 +933,10 @@ bool attention_supported(uint32_t qh, uint32_t kvh, uint32_t hd, uint64_t total)
 // every launch is per query head.
 bool attention_per_kv(uint32_t G, uint32_t hd) { return hd == 256 ? G == 1 || G == 2 || G == 4 : G >= 1 && G <= 8; }
 
+bool attention_may_go_plain(uint32_t G, uint32_t hd) {
+  return hd == 96 || (G & (G - 1)) != 0 || !attention_per_kv(G, hd);
+}
+
 // Chunks per KV head: 64 positions each while that keeps the launch within
 // about 256 workgroups (one per CU), longer chunks beyond (at most
 // ATT_MAX_SPLITS chunks of at most ATT_MAX_CHUNK positions).  Timed on

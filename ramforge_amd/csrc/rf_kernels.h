@@ -246,6 +246,11 @@ bool attention_supported(uint32_t qh, uint32_t kvh, uint32_t hd, uint64_t total_
 // It has a form with the G = qh / kvh query heads of a KV head in one
 // workgroup (else its launches are per query head, per_q).
 bool attention_per_kv(uint32_t G, uint32_t hd);
+// Group sizes other than 1, 2, 4 and 8, head_dim 96 and per-query-head shapes:
+// the any-shape kernel served them first, in workspaces (and prompts in
+// budgets) that hold no chunk records, and still does where those are refused.
+// The other shapes' refusals are their callers' errors.
+bool attention_may_go_plain(uint32_t G, uint32_t hd);
 
 // Batched prefill (rf_prefill.hip): Y[t][r] = sum_k W[r][k] X[t][k] for up to
 // MM_MAX_TOKENS tokens on the packed layout, on the matrix cores, with split-K

@@ -1977,12 +1977,9 @@ int32_t enqueue_prefill_layer(rf_model* m, size_t li, uint64_t pos0, uint64_t nt
 
 // Whether a prompt without room for its workspace runs by single forwards.  A
 // refused workspace is the caller's error, who sizes the budget by it: single
-// forwards take ten times as long.  Group sizes other than 1, 2, 4 and 8 and
-// head_dim 96 have had single forwards only, so budgets that hold no workspace
-// are in use with them.
+// forwards take ten times as long.
 bool prefill_optional(const rf_model* m) {
-  const uint64_t G = m->cfg.head_count / m->cfg.head_count_kv, hd = m->cfg.head_dim;
-  return hd == 96 || (G & (G - 1)) != 0 || !attention_per_kv((uint32_t)G, (uint32_t)hd);
+  return attention_may_go_plain((uint32_t)(m->cfg.head_count / m->cfg.head_count_kv), (uint32_t)m->cfg.head_dim);
 }
 
 // The chunks of a prompt through the layers; the workspace is there.

@@ -1137,6 +1137,11 @@ int32_t rf_attention_decode(rf_ctx* ctx, const float* q, const float* kh, const 
   if (rc) return rc;
   hipStream_t st = pick_stream(ctx, s);
   rc = ensure_workspace(ctx, ctx->attn_ws, "workspace:attention", ws_bytes, st);
+  if (rc && fast && attention_may_go_plain(qh / kvh, hd)) {  // no room for the chunk records: the score rows may fit
+    fast = false;
+    a.nsplit = 1;
+    rc = ensure_workspace(ctx, ctx->attn_ws, "workspace:attention", (uint64_t)qh * (hist + 1) * 4, st);
+  }
   if (rc) return rc;
   a.ws = static_cast<float*>(ctx->attn_ws.ptr);
   return attention_launch(a, fast, st);

@@ -47,6 +47,35 @@ def test_attention_groups_equal_the_any_shape_kernel(ctx, qh, kvh, hd):
         x.free()
 
 
+@pytest.mark.parametrize("qh,kvh,hd,runs", [(40, 8, 128, True), (32, 8, 128, False)])
+def test_attention_groups_without_room_for_the_records(qh, kvh, hd, runs):
+    """A workspace that holds the score rows of 101 positions and not the chunk
+    records, and that a capture cannot grow: five heads per KV head run the
+    any-shape kernel (f32 sums in another order: 1e-5 of the largest output),
+    four heads are refused."""
+    rf = _rf()
+    hist = 100
+    rng = np.random.default_rng(qh)
+    with rf.Context(0) as c:
+        dev = [c.array(rng.normal(0, 1, n).astype(np.float32))
+               for n in (qh * hd, hist * kvh * hd, hist * kvh * hd, kvh * hd, kvh * hd)]
+        out = c.empty((qh * hd,))
+        rf.attention_checked(c, *dev, 10, qh, kvh, hd, out=out)  # one chunk: no records
+        if not runs:
+            with pytest.raises(rf.RamforgeError, match="during graph capture"):
+                with c.capture():
+                    rf.attention_checked(c, *dev, hist, qh, kvh, hd, out=out)
+            return
+        with c.capture() as cap:
+            rf.attention_checked(c, *dev, hist, qh, kvh, hd, out=out)
+        cap.graph.replay(2)
+        got = out.numpy()
+        cap.graph.close()
+        rf.attention_checked(c, *dev, hist, qh, kvh, hd, out=out)
+        ref = out.numpy()
+    assert np.max(np.abs(got - ref)) <= 1e-5 * np.abs(ref).max() and not np.array_equal(got, ref)
+
+
 @pytest.mark.parametrize("qh,kvh,hd,kind", [(12, 2, 128, "q4"), (6, 2, 64, "q8"), (5, 1, 96, "q8"),
                                             (32, 2, 64, "q8"), (6, 1, 256, "q8"), (7, 1, 64, "q8"),
                                             (14, 2, 128, "q4")])
